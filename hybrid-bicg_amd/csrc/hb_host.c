@@ -128,8 +128,13 @@ struct hbicg_plan {
     double *aa, *ba, *wa, *pi, *eta, *zeta, *coef, *ccoef, *grow, *part, *trace, *p_snap;
     int *stop, *stop_iter, *act_len, *flist, *fpos, *switch_k, *switch_to;
     hb_state *st;
-    int *flag_host;      /* pinned: {done, k} */
+    int *flag_host;      /* pinned: {done, k, res_fail, ks} */
     hipEvent_t ev[2], t0, t1;
+    /* resident form: layout, ring of p, logs, mailboxes (hb_resident.hip) */
+    int *rend;
+    unsigned short *rpres;
+    double *rdia, *pring, *drlog, *qqlog;
+    unsigned long long *mail;
     /* graph of one chunk, captured for a given x_set pointer */
     hipGraphExec_t gexec;
     hipGraph_t graph_obj;
@@ -194,7 +199,8 @@ void hbicg_plan_destroy(hbicg_plan *pl)
     void *bufs[] = {pl->blk, pl->col16, pl->cflag, pl->rhat, pl->rring, pl->qring, pl->s, pl->y, pl->p_set, pl->x_host_buf,
                     pl->b_buf, pl->sigma, pl->aa, pl->ba, pl->wa, pl->pi, pl->eta, pl->zeta,
                     pl->coef, pl->ccoef, pl->grow, pl->part, pl->trace, pl->p_snap, pl->vidx, pl->vdict, pl->col16p, pl->tpad, pl->dtile, pl->doff, pl->didx, pl->dval, pl->pval, pl->pcol, pl->pptr, pl->pblk, pl->flush_log, pl->stop, pl->stop_iter, pl->act_len, pl->flist, pl->fpos,
-                    pl->switch_k, pl->switch_to, pl->st};
+                    pl->switch_k, pl->switch_to, pl->st, pl->rend, pl->rpres, pl->rdia,
+                    pl->pring, pl->drlog, pl->qqlog, pl->mail};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
         if (bufs[i]) hipFree(bufs[i]);
     if (pl->flag_host) hipHostFree(pl->flag_host);
@@ -636,6 +642,96 @@ done:
     return rc;
 }
 
+/* The resident form of the default order (hb_resident.hip), where it fits:
+ * every SpMV tile is 256 rows (at most 8 entries a row on average), the
+ * matrix has at most HB_DIAG_K diagonals, columns ascending, and the rows fit
+ * the compute units (8192 each).  Elsewhere the plan keeps the
+ * launch-per-phase kernels.  A launch runs at most res_C iterations, whose
+ * p stay in a ring (256 MiB of it, 32 slots at least): a window the growth
+ * guard closes in the middle needs the p of its successor's first iteration. */
+static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
+{
+    int rc = 0, cus = 0, SB = 0, E = 0, lcw = 0, bad = 0, K = 0;
+    int *work = NULL, *host = NULL;
+    hb_dev *d = &pl->dev;
+    const int n = pl->n, nblk = pl->nblk;
+    if (nblk != (n + HB_BLOCK - 1) / HB_BLOCK) return 0;
+    for (int t = 0; t < nblk; ++t)
+        if (hblk[t] != (unsigned)t * HB_BLOCK) return 0;
+    HIPCK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device));
+    const int G = hb_k_res_shape(nblk, cus, &SB, &E, &lcw);
+    if (G <= 0) return 0;
+    /* tile diagonals | their number | bad; then the value patterns */
+    const size_t words = (size_t)nblk * (HB_DIAG_K + 1) + 1;
+    work = (int *)dalloc(words * sizeof(int) + 4 * HB_DIAG_K * 8, &rc);
+    host = (int *)malloc(words * sizeof(int));
+    if (!host) rc = HBICG_E_NOMEM;
+    if (rc) goto fail;
+    int *const dK = work + (size_t)nblk * HB_DIAG_K, *const dbad = dK + nblk;
+    HIPCK(hipMemcpyAsync(dbad, &bad, sizeof bad, hipMemcpyHostToDevice, pl->stream));
+    if (hb_k_res_scan(d, dK, work, dbad, pl->stream) != 0) { rc = HBICG_E_HIP; goto fail; }
+    HIPCK(hipMemcpyAsync(host, work, words * sizeof(int), hipMemcpyDeviceToHost, pl->stream));
+    HIPCK(hipStreamSynchronize(pl->stream));
+    if (host[words - 1]) goto fail;
+    int off[HB_DIAG_K + 1];
+    for (int t = 0; t < nblk; ++t)
+        for (int s = 0; s < host[(size_t)nblk * HB_DIAG_K + t]; ++s) {
+            const int o = host[(size_t)t * HB_DIAG_K + s];
+            int at = 0;
+            while (at < K && off[at] < o) ++at;
+            if (at < K && off[at] == o) continue;
+            if (K == HB_DIAG_K) goto fail;
+            for (int u = K; u > at; --u) off[u] = off[u - 1];
+            off[at] = o;
+            ++K;
+        }
+    if (K < 1) goto fail;
+    int KT = K <= 8 ? 8 : HB_DIAG_K;
+    if ((K == 5 || K == 7) && off[K / 2] == 0) KT = K;
+    pl->rpres = (unsigned short *)dalloc((size_t)n * 2, &rc);
+    if (rc) goto fail;
+    d->res_K = K;
+    d->res_KT = KT;
+    for (int j = 0; j < HB_DIAG_K; ++j) d->res_off[j] = j < K ? off[j] : 0;
+    uint64_t pat[2 * HB_DIAG_K];
+    for (int j = 0; j < HB_DIAG_K; ++j) {
+        pat[j] = ~(uint64_t)0;
+        pat[HB_DIAG_K + j] = 0;
+    }
+    unsigned long long *const dpat = (unsigned long long *)(((uintptr_t)(dbad + 1) + 7) & ~(uintptr_t)7);
+    HIPCK(hipMemcpyAsync(dpat, pat, sizeof pat, hipMemcpyHostToDevice, pl->stream));
+    if (hb_k_res_bits(d, pl->rpres, dpat, dpat + HB_DIAG_K, pl->stream) != 0) { rc = HBICG_E_HIP; goto fail; }
+    HIPCK(hipMemcpyAsync(pat, dpat, sizeof pat, hipMemcpyDeviceToHost, pl->stream));
+    HIPCK(hipStreamSynchronize(pl->stream));
+    /* one value per diagonal only where the plan may keep values */
+    int full = d->nvdict == 0;
+    for (int j = 0; j < K; ++j) {
+        if (pat[j] != pat[HB_DIAG_K + j]) full = 1;
+        memcpy(&d->res_val[j], &pat[j], 8);
+    }
+    for (int j = full ? 0 : K; j < HB_DIAG_K; ++j) d->res_val[j] = 0.0;
+    int C = (int)(((size_t)256 << 20) / ((size_t)n * 8));
+    if (C < 32) C = 32;
+    if (C > HB_RES_CMAX) C = HB_RES_CMAX;
+    if (C > pl->W) C = pl->W;
+    pl->rend = (int *)dalloc(2 * sizeof(int), &rc);
+    pl->pring = (double *)dalloc((size_t)(C + 1) * n * 8, &rc);
+    pl->drlog = (double *)dalloc((size_t)pl->cap * 8, &rc);
+    pl->qqlog = (double *)dalloc((size_t)pl->cap * 8, &rc);
+    pl->mail = (unsigned long long *)dalloc((size_t)3 * 2048 * 8 + (size_t)G * 64, &rc);
+    if (full) pl->rdia = (double *)dalloc((size_t)nblk * KT * HB_BLOCK * 8, &rc);
+    if (rc) goto fail;
+    d->rpres = pl->rpres; d->rend = pl->rend; d->rdia = pl->rdia; d->pring = pl->pring;
+    d->drlog = pl->drlog; d->qqlog = pl->qqlog; d->mail = pl->mail;
+    d->res_SB = SB; d->res_E = E; d->res_lcw = lcw; d->res_C = C; d->res_P = C + 1; d->res_full = full;
+    d->res_join = join;
+    d->res_G = G;
+fail:
+    if (work) hipFree(work);
+    free(host);
+    return rc;
+}
+
 /* w_alloc: ring storage for windows up to this (the batched solver's
  * autotuner); w_cap: the largest window the plan may choose; allow_vi: the
  * SpMV may read the matrix through a value table (params.value_index);
@@ -768,7 +864,7 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
     if (rc) goto fail;
     /* unused combined-coefficient columns stay finite */
     HIPCK(hipMemset(pl->ccoef, 0, ccn * 8));
-    HIPCK(hipHostMalloc((void **)&pl->flag_host, 2 * sizeof(int), hipHostMallocDefault));
+    HIPCK(hipHostMalloc((void **)&pl->flag_host, 4 * sizeof(int), hipHostMallocDefault));
     HIPCK(hipEventCreateWithFlags(&pl->ev[0], hipEventDisableTiming));
     HIPCK(hipEventCreateWithFlags(&pl->ev[1], hipEventDisableTiming));
     HIPCK(hipEventCreate(&pl->t0));
@@ -855,10 +951,10 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
 
     /* alpha~'s finalize joins SpMV 2 where that launch forms q at its
      * gathered columns in one pass */
-    d->fused_a = d->fused && !d->q_unfused && d->npanel <= 1 && (p->fused == 1 || p->fused == 3);
+    d->fused_a = d->fused && !d->q_unfused && d->npanel <= 1 && (p->fused == 1 || p->fused == 3 || p->fused == 4);
     /* the scalar stage joins the shift kernel (level 1), whose tiles then
      * walk the seed p update and the flush tiles grid-stride */
-    d->fused_s = d->fused && p->fused == 1;
+    d->fused_s = d->fused && (p->fused == 1 || p->fused == 4);
     if (d->fused_s) {
         d->shift_tw = hb_k_shift_stage_tiles(d->shift_gx, M, pl->device);
         if (d->shift_tw < 0) { rc = HBICG_E_HIP; goto fail; }
@@ -866,6 +962,11 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
          * launch of its own (the five-launch form, bitwise the same) */
         if (d->shift_tw == 0) d->fused_s = 0;
     }
+    /* the resident form: default launches, windows long enough for a launch
+     * to run a useful number of iterations */
+    if (d->fused && (p->fused == 1 || p->fused == 4) && !pl->profile && d->npanel <= 1 && pl->W >= HB_RES_WMIN &&
+        (rc = setup_resident(pl, hblk, p->fused == 4 ? 0 : HB_RES_JOIN)) != 0)
+        goto fail;
     if (a_on_device) free(hptr);
     free(hblk);
     return pl;
@@ -1000,10 +1101,60 @@ fail:
     return rc;
 }
 
+/* Rounds of the resident form: up to res_C iterations of the seed process,
+ * the shifts over them, and the window flush when one is due.  Where a round
+ * holds few iterations the host reads its flags while the next one runs;
+ * where one or two rounds are the whole solve it waits for them, which takes
+ * about the same time as the five empty launches of a round too many (25 us)
+ * and leaves the GPU to others.  Returns 0 at the end of the
+ * solve, 1 when the launch-per-phase kernels have to take over (a launch
+ * could not get all its workgroups resident), or an error. */
+static int run_resident(hbicg_plan *pl)
+{
+    int rc = 0, launched = 0, prev = -1, fail = 0;
+    const hb_dev *d = &pl->dev;
+    const int ahead = d->res_C < 256;
+    for (int i = 0; i < 4; ++i) pl->flag_host[i] = 0;
+    if (d->res_full && hb_k_res_fill(d, pl->stream) != 0) return HBICG_E_HIP;
+    while (launched <= 2 * pl->cap + 8) {   /* every other round advances an iteration at least */
+        if (hb_k_res_iterations(d, pl->stream) != 0 || hb_k_res_flush(d, pl->stream) != 0 ||
+            hb_k_publish(d, pl->flag_host, pl->stream) != 0)
+            return HBICG_E_HIP;
+        const int cur = launched & 1;
+        HIPCK(hipEventRecord(pl->ev[cur], pl->stream));
+        ++launched;
+        if (!ahead) prev = cur;
+        if (prev >= 0) {
+            HIPCK(hipEventSynchronize(pl->ev[prev]));
+            if (__atomic_load_n(&pl->flag_host[0], __ATOMIC_ACQUIRE)) break;
+            if ((fail = __atomic_load_n(&pl->flag_host[2], __ATOMIC_ACQUIRE)) != 0) break;
+        }
+        prev = cur;
+    }
+    HIPCK(hipStreamSynchronize(pl->stream));
+    if (!fail || pl->flag_host[0]) return 0;
+    /* the shifts catch up with what the seed process has run */
+    for (int i = 0; i <= pl->cap && !pl->flag_host[0] && pl->flag_host[1] != pl->flag_host[3]; ++i) {
+        if (hb_k_res_stage(d, pl->stream) != 0 || hb_k_res_flush(d, pl->stream) != 0 ||
+            hb_k_publish(d, pl->flag_host, pl->stream) != 0)
+            return HBICG_E_HIP;
+        HIPCK(hipStreamSynchronize(pl->stream));
+    }
+    if (pl->flag_host[0]) return 0;
+    return hb_k_res_leave(d, pl->stream) != 0 ? HBICG_E_HIP : 1;
+fail:
+    return rc;
+}
+
 static int run_loop(hbicg_plan *pl)
 {
     int rc = 0;
     if (pl->profile) return run_loop_profiled(pl);
+    if (pl->dev.res_G) {
+        if ((rc = run_resident(pl)) <= 0) return rc;
+        rc = 0;
+        pl->dev.res_G = 0;   /* for the rest of this solve */
+    }
     if (pl->graph && (rc = capture_graph(pl)) != 0) return rc;
     pl->flag_host[0] = 0;
     pl->flag_host[1] = 0;
@@ -1071,11 +1222,13 @@ int hbicg_plan_solve(hbicg_plan *pl, const double *b, const double *sigma, int s
     }
     if (pl->flush_log) HIPCK(hipMemsetAsync(pl->flush_log, 0, (size_t)pl->cap * sizeof(int), pl->stream));
     if (hb_k_init(&pl->dev, pl->stream) != 0) { rc = HBICG_E_HIP; goto fail; }
+    const int res_G = pl->dev.res_G;
     if ((rc = run_loop(pl)) != 0) goto fail;
     /* profiled solves time the finalize: it holds the last window flush
      * when the shift kernel runs the scalar stage */
     if (pl->profile) HIPCK(hipEventRecord(pl->pev[0], pl->stream));
     if (hb_k_finalize(&pl->dev, pl->stream) != 0) { rc = HBICG_E_HIP; goto fail; }
+    pl->dev.res_G = res_G;
     if (pl->profile) HIPCK(hipEventRecord(pl->pev[1], pl->stream));
     HIPCK(hipEventRecord(pl->t1, pl->stream));
 

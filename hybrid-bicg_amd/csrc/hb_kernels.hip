@@ -43,37 +43,7 @@
 #include <math.h>
 #include "hb_shared.h"
 #include "hb_launch.h"
-
-#define DEV __device__ __forceinline__
-
-typedef double dbl2 __attribute__((ext_vector_type(2)));
-
-/* Constant address space: the compiler takes what is read through it as
- * unchanged for the rest of the launch, and a wave-uniform address there
- * becomes a scalar load. */
-#define HB_K __attribute__((address_space(4)))
-
-/* p, from here to the end of the launch read-only, as constant memory.  The
- * empty asm makes the returned pointer unknown to the compiler until this
- * point, so no read through it moves above what comes before (a wait for
- * the data in the same launch).  Without it a kernel with a barrier or an
- * atomic anywhere before the reads loses their scalar loads: the compiler
- * cannot show that nothing in between stored to them, and makes every
- * uniform read a vector load. */
-template <typename T>
-DEV const HB_K T *read_only(const T *p)
-{
-    asm volatile("" : "+s"(p));
-    return (const HB_K T *)p;
-}
-
-/* ---- reductions ----------------------------------------------------------- */
-DEV double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
+#include "hb_device.h"
 
 /* Sums a and b over the workgroup; the result is valid in thread 0. */
 DEV void block_sum2(double &a, double &b)
@@ -143,104 +113,6 @@ DEV double serial_dot(const double *x, const double *y, int n, double *lds)
     }
     return acc;
 }
-
-/* ---- values handed between the workgroups of one launch ---------------------
- * A workgroup dispatched first computes a value the launch's other
- * workgroups need.  It stores it with an agent-scope relaxed atomic store (a
- * write-through store, sc1, on gfx950) into a mailbox that holds
- * HB_MAIL_EMPTY until then; the others poll it with agent-scope relaxed
- * atomic loads (sc1), which read past any stale cache line.  Every word
- * that crosses workgroups inside a launch moves this way, so no L2
- * write-back or invalidate (what an agent-scope release or acquire costs)
- * is needed.  The first workgroups of a grid are dispatched before the
- * later ones (in order on each XCD), so the publisher is always running
- * when a waiter spins; the spin is bounded all the same (about 0.5 s), and
- * a waiter that gives up sets HB_ST_SYNC_TIMEOUT and goes on instead of
- * hanging; every later waiter sees the bit and does not wait at all. */
-#define HB_SPIN_LIMIT (1 << 17)
-
-/* a waiter polls the status word too: once one has timed out, none waits */
-DEV bool sync_timed_out(hb_state *st)
-{
-    return (__hip_atomic_load(&st->status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & HB_ST_SYNC_TIMEOUT) != 0;
-}
-
-DEV void mail_put(unsigned long long *slot, unsigned long long v)
-{
-    __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-DEV void mail_put_d(unsigned long long *slot, double v)
-{
-    mail_put(slot, (unsigned long long)__double_as_longlong(v));
-}
-
-/* the published word, polled by the calling thread alone (HB_MAIL_EMPTY
- * after a time-out) */
-DEV unsigned long long mail_poll_bits(unsigned long long *slot, hb_state *st)
-{
-    unsigned long long v;
-    for (int spins = 0;; ++spins) {
-        v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (v != HB_MAIL_EMPTY) break;
-        if (spins == HB_SPIN_LIMIT || ((spins & 255) == 255 && sync_timed_out(st))) {
-            atomicOr(&st->status, HB_ST_SYNC_TIMEOUT);
-            break;
-        }
-        /* a few hundred cycles between polls: thousands of resident
-         * workgroups poll one word, and the publisher needs the memory
-         * system more than they do */
-        __builtin_amdgcn_s_sleep(8);
-    }
-    return v;
-}
-
-DEV double mail_poll(unsigned long long *slot, hb_state *st)
-{
-    return __longlong_as_double((long long)mail_poll_bits(slot, st));
-}
-
-/* the published double; thread 0 of the workgroup waits, every thread gets it */
-DEV double mail_wait(unsigned long long *slot, hb_state *st)
-{
-    __shared__ double sh_v;
-    if (threadIdx.x == 0) sh_v = mail_poll(slot, st);
-    __syncthreads();
-    return sh_v;
-}
-
-/* the published word, to every thread of the workgroup */
-DEV unsigned long long mail_wait_bits(unsigned long long *slot, hb_state *st)
-{
-    __shared__ unsigned long long sh_u;
-    if (threadIdx.x == 0) sh_u = mail_poll_bits(slot, st);
-    __syncthreads();
-    return sh_u;
-}
-
-/* a value the kernel's other workgroups read before the launch ends */
-template <bool PUB>
-DEV void store_pub(double *p, double v)
-{
-    if (PUB) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *p = v;
-}
-
-template <bool PUB>
-DEV void store_pub(int *p, int v)
-{
-    if (PUB) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *p = v;
-}
-
-/* a word another workgroup of the launch stored with store_pub<true> */
-DEV int load_pub(const int *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-DEV size_t off(int j, int n) { return (size_t)j * (size_t)n; }
-#define PI(d, j, i) ((d).pi[(size_t)(j) * (size_t)(d).cap + (size_t)(i)])
 
 /* ---- SpMV ------------------------------------------------------------------
  * Tile b owns rows [blk[b], blk[b+1]).  When their nonzeros fit in LDS
@@ -750,17 +622,6 @@ DEV void spmv_tile(const hb_dev &d, unsigned b)
                                                              nullptr, d.rring, d.s, d.rhat, d.y, d.qring, d.part2,
                                                              0.0, d.vidx, d.col16p, d.tpad, d.vdict, d.dtile,
                                                              d.doff, d.didx, d.dval);
-}
-
-/* Workgroup b runs on XCD b % 8 (the dispatcher deals workgroups round
- * robin over the eight XCDs, each with its own L2).  Tile order: XCD x gets
- * the contiguous tiles [start(x), start(x+1)), so a tile's column halo (the
- * rows around it, and the rows a plane away for stencils) was mostly
- * fetched into the same L2 by its neighbours.  A bijection on 0 .. nb-1. */
-DEV unsigned xcd_tile(unsigned b, unsigned nb)
-{
-    const unsigned q = nb / 8, r = nb % 8, x = b % 8;
-    return x * q + min(x, r) + b / 8;
 }
 
 template <int MODE, bool EXACT, bool VI, bool UNF = false, bool CD = false>
@@ -1771,6 +1632,56 @@ __global__ __launch_bounds__(HB_BLOCK) void k_flush_coef(hb_dev d)
     flush_coef_body(d, blockIdx.x, d.coef, d.ccoef);
 }
 
+/* flush_coef_body for the resident form, a launch of its own: one component
+ * per thread (workgroup y of a position takes components 256 y - 1 ...), the
+ * window's steps walked together by the workgroup so that a step's six
+ * coefficients are uniform reads.  A component's walk starts where it first
+ * is not zero; lanes before that keep their zeros. */
+__global__ __launch_bounds__(HB_BLOCK) void k_res_coef(hb_dev d)
+{
+    const hb_state *st = d.st;
+    const int pos = blockIdx.x;
+    if (!st->res_flush || pos >= st->flush_cnt) return;
+    const int M = d.M, W = d.W, L = st->flush_len, ntail = st->flush_tail;
+    const int Lc = L - ntail, lv = d.act_len[pos], nb = min(lv, Lc);
+    const int kc = (int)(blockIdx.y * HB_BLOCK + threadIdx.x) - 1;   /* -1: the p_j component */
+    const int c0 = (int)(blockIdx.y * HB_BLOCK) - 1;
+    if (c0 > 2 * Lc) return;
+    const HB_K double *coef = read_only((const double *)d.coef);
+    double *blk = d.ccoef + (size_t)(pos / HB_UG) * (size_t)HB_CC_ROWS(W) * (2 * HB_UG);
+    const bool pch = kc < 0;
+    if (pch && Lc < L) {
+        const HB_K double *c = coef + ((size_t)(L - 1) * M + pos) * 6;
+        const bool on = lv == L;
+        const int base = (2 * W + 2) * (2 * HB_UG) + pos % HB_UG;
+#pragma unroll
+        for (int e = 0; e < 6; ++e)
+            blk[base + (e / 2) * (2 * HB_UG) + (e % 2) * HB_UG] = on ? c[e] : e == 4 ? 1.0 : 0.0;
+    }
+    const int from = kc > 0 ? (kc - 1) / 2 : 0;
+    const int wave_c = __builtin_amdgcn_readfirstlane(kc);   /* the wave's first component */
+    dd xk = {0.0, 0.0}, pk = {pch ? 1.0 : 0.0, 0.0};
+    for (int b = wave_c > 0 ? (wave_c - 1) / 2 : 0; b < nb; ++b) {
+        const HB_K double *c = coef + ((size_t)b * M + pos) * 6;
+        const double k0 = c[0], k1 = c[1], k2 = c[2], k3 = c[3], k4 = c[4], k5 = c[5];
+        if (b >= from) {
+            dd xn = dd_add(xk, dd_mul(pk, k1));
+            dd tp = pk;
+            if (kc == 2 * b + 1) { xn = dd_add(xn, k0); tp = dd_add(tp, k2); }
+            if (kc == 2 * b) tp = dd_add(tp, k3);
+            dd pn = dd_mul(tp, k4);
+            if (kc == 2 * b + 2) pn = dd_add(pn, k5);
+            xk = xn;
+            pk = pn;
+        }
+    }
+    if (kc <= 2 * Lc) {
+        const int row = 1 + kc;
+        blk[(size_t)row * (2 * HB_UG) + pos % HB_UG] = xk.hi + xk.lo;
+        blk[(size_t)row * (2 * HB_UG) + HB_UG + pos % HB_UG] = pk.hi + pk.lo;
+    }
+}
+
 /* The window a flush applies: its first iteration, list length, regrouped
  * iterations, tail flag and the seed's list position, uniform across the
  * workgroup (read once by the caller, kept in scalar registers). */
@@ -2245,7 +2156,7 @@ DEV void shift_stage_tiles(const hb_dev &d, int t, int T)
 }
 
 /* The solve's last window flush (x_j only) after the iteration loop, when the
- * shift kernel runs the scalar stage: that iteration's stage marked it
+ * shift kernel runs the scalar stage (or in the resident form): that iteration's stage marked it
  * (flush, flush_xonly) and its coefficient workgroups formed the combined
  * coefficients.  One workgroup per 256-element tile. */
 __global__ __launch_bounds__(HB_BLOCK) void k_flush_final(hb_dev d)
@@ -2254,6 +2165,21 @@ __global__ __launch_bounds__(HB_BLOCK) void k_flush_final(hb_dev d)
     if (!st->flush || !st->flush_xonly) return;
     const hb_fl fw = flush_window(st->flush_k0, st->flush_cnt, st->flush_len, st->flush_tail, st->win_seedpos);
     flush_apply_x2<HB_UG>(d, blockIdx.x, fw, d.x_set, d.p_set, d.rring, d.qring, d.ccoef, d.flist);
+}
+
+/* A window flush of the resident form that is not the solve's last. */
+__global__ __launch_bounds__(HB_BLOCK) void k_res_flush(hb_dev d)
+{
+    const hb_state *st = d.st;
+    if (st->res_flush != 1) return;
+    const hb_fl fw = flush_window(st->flush_k0, st->flush_cnt, st->flush_len, st->flush_tail, st->win_seedpos);
+    flush_apply<HB_UG>(d, blockIdx.x, fw, d.x_set, d.p_set, d.rring, d.qring, d.ccoef, d.flist);
+    const int ks = st->res_snap;
+    if (ks) {
+        __syncthreads();   /* the tile's old snapshot has been read */
+        const int i = blockIdx.x * HB_BLOCK + threadIdx.x;
+        if (i < d.n) d.p_snap[i] = d.pring[off(ks % d.res_P, d.n) + i];
+    }
 }
 
 /* Shift kernel with the scalar stage (default mode, fused level 1):
@@ -2357,6 +2283,15 @@ DEV void init_fin_body(const hb_dev &d)
         st->coef_ready = 0;
         st->mail_w = HB_MAIL_EMPTY;
         st->mail_a = HB_MAIL_EMPTY;
+        st->ks = 1;
+        st->res_fresh = 1;
+        st->res_flush = 0;
+        st->res_snap = 0;
+        st->res_fail = 0;
+        if (d.res_G) {
+            d.rend[0] = 0;
+            d.rend[1] = 0;
+        }
     }
 }
 
@@ -2385,8 +2320,10 @@ __global__ __launch_bounds__(HB_BLOCK) void k_finalize(hb_dev d)
 __global__ void k_publish(const hb_state *st, int *flag)
 {
     if (threadIdx.x == 0) {
-        flag[0] = st->done;
         flag[1] = st->k;
+        flag[2] = st->res_fail;
+        flag[3] = st->ks;
+        flag[0] = st->done;
         __threadfence_system();
     }
 }
@@ -2837,8 +2774,15 @@ int hb_k_publish(const hb_dev *d, int *flag_dev, hipStream_t s)
 
 int hb_k_finalize(const hb_dev *d, hipStream_t s)
 {
-    if (d->fused_s) hipLaunchKernelGGL(k_flush_final, dim3(d->shift_gx), dim3(HB_BLOCK), 0, s, *d);
+    if (d->fused_s || d->res_G) hipLaunchKernelGGL(k_flush_final, dim3(d->shift_gx), dim3(HB_BLOCK), 0, s, *d);
     hipLaunchKernelGGL(k_finalize, dim3(d->vec_grid), dim3(HB_BLOCK), 0, s, *d);
+    return (int)hipGetLastError();
+}
+
+int hb_k_res_flush(const hb_dev *d, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_res_coef, dim3(d->M, (2 * d->W + 2 + HB_BLOCK - 1) / HB_BLOCK), dim3(HB_BLOCK), 0, s, *d);
+    hipLaunchKernelGGL(k_res_flush, dim3(d->shift_gx), dim3(HB_BLOCK), 0, s, *d);
     return (int)hipGetLastError();
 }
 

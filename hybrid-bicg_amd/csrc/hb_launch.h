@@ -48,7 +48,7 @@ int hb_k_shift_stage_tiles(int n_tiles, int M, int device);
 #define HB_NSTAGE       8
 int hb_k_stage(const hb_dev *d, int stage, hipStream_t s);
 
-/* Copies {done, k} of the device state into host-visible memory. */
+/* Copies {done, k, res_fail, ks} of the device state into host-visible memory. */
 int hb_k_publish(const hb_dev *d, int *flag_dev, hipStream_t s);
 
 /* After the iteration loop: the solve's last, x-only window flush when the
@@ -71,6 +71,28 @@ int hb_k_compress_cols(const hb_dev *d, short *col16, unsigned *cflag, hipStream
 
 /* y = A x + shift*x through the row-binned SpMV (exact: row-sequential sums). */
 int hb_k_spmv(const hb_dev *d, const double *x, double *y, double shift, hipStream_t s);
+
+/* ---- resident form (hb_resident.hip) ---- */
+/* Workgroups (at most one per compute unit) for nblk tiles of 256 rows, 0
+ * where the rows do not fit, and how the tiles are dealt (hb_dev). */
+int hb_k_res_shape(int nblk, int cus, int *SB, int *E, int *lcw);
+/* Each tile's diagonals (tK, toff[16 a tile]); bad set where there are more
+ * than HB_DIAG_K, or columns that do not ascend. */
+int hb_k_res_scan(const hb_dev *d, int *tK, int *toff, int *bad, hipStream_t s);
+/* Presence bits on d->res_off, and the least and greatest bit pattern of each
+ * diagonal's values (lo all ones, hi zero before). */
+int hb_k_res_bits(const hb_dev *d, unsigned short *pres, unsigned long long *lo, unsigned long long *hi,
+                  hipStream_t s);
+/* rdia from val, at the start of a solve. */
+int hb_k_res_fill(const hb_dev *d, hipStream_t s);
+/* Up to res_C iterations of the seed process, then the shifts over them. */
+int hb_k_res_iterations(const hb_dev *d, hipStream_t s);
+/* The shifts alone, over iterations that have run. */
+int hb_k_res_stage(const hb_dev *d, hipStream_t s);
+/* The window flush the stage decided, when it did (hb_kernels.hip). */
+int hb_k_res_flush(const hb_dev *d, hipStream_t s);
+/* Hands a solve over to hb_k_iteration. */
+int hb_k_res_leave(const hb_dev *d, hipStream_t s);
 
 /* Batched counterparts: each launch covers the tiles of every problem of
  * the batch; done problems return at once. */

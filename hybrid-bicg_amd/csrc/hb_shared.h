@@ -27,6 +27,9 @@ extern "C" {
 /* default column-panel width of the seed SpMVs: 2 MiB of x, half an XCD's L2 */
 #define HB_PANEL_COLS 262144
 #define HB_MAXPANEL   32      /* most panels; wider panels beyond               */
+#define HB_RES_WMIN   16      /* shortest window the resident form is used with */
+#define HB_RES_JOIN   16384   /* polls a resident workgroup waits for the others, about 15 ms */
+#define HB_RES_CMAX   512     /* most iterations of a resident launch          */
 #define HB_RESID_PAIRS  65536 /* most partial pairs of one true-residual evaluation */
 
 /* Error bits in hb_state.status */
@@ -103,6 +106,15 @@ typedef struct hb_state {
                           the stage rescales the archives at a switch)         */
     int pu_live;       /* 1 once omega~'s finalize ran this iteration (SpMV 1
                           clears it): the shift kernel's tiles have work      */
+    /* the resident form (hb_resident.hip): the seed process runs ahead of the
+     * shifts, which k counts */
+    int ks;            /* iteration the seed process runs next                */
+    int res_fresh;     /* 1: the seed's p starts from p_set (first iteration,
+                          seed switch), else from the ring of p               */
+    int res_flush;     /* the last stage closed a window: 1 x_j and p_j, 2 x_j only */
+    int res_snap;      /* the window that follows has run already: iteration
+                          whose p the flush keeps as its snapshot, else 0     */
+    int res_fail;      /* a launch could not get all its workgroups resident  */
 } hb_state;
 
 /* Every pointer below addresses global device memory.  Device code sees
@@ -201,6 +213,22 @@ typedef struct hb_dev {
                                   kernel applied a window flush, else NULL       */
     HB_G double *trace;        /* [cap][M] estimated residual per iteration and shift,
                                   -1 once stopped (NULL: not recorded)     */
+    /* resident form of the default order (res_G > 0), see hb_resident.hip */
+    int res_G, res_SB, res_E;  /* workgroups; tiles per group of 256 threads: SB times E */
+    int res_lcw;               /* log2 of the partial-sum columns a workgroup owns */
+    int res_C, res_P;          /* most iterations of a launch; slots of the ring of p */
+    int res_K, res_KT;         /* diagonals of the matrix; of the kernel's form (the rest
+                                  are empty)                                 */
+    int res_full;              /* 1: values per row (rdia), 0: per diagonal (res_val) */
+    int res_join;              /* polls a workgroup waits for the others to become resident */
+    int res_off[HB_DIAG_K];    /* the diagonals, column - row, ascending     */
+    double res_val[HB_DIAG_K];
+    HB_G const unsigned short *rpres; /* [n] presence bits                   */
+    HB_G double *rdia;         /* [nblk][res_KT][256]                        */
+    HB_G double *pring;        /* [res_P][n] p at the start of iteration k in slot k mod res_P */
+    HB_G double *drlog, *qqlog;/* [cap] (r,r) and (q,q) of every iteration   */
+    HB_G unsigned long long *mail; /* mailboxes and epoch flags of a launch  */
+    HB_G int *rend;            /* workgroups arrived; 1 go, 2 given up       */
     HB_G hb_state *st;
     HB_G const double *b_in;   /* right-hand side read by the initialisation */
     int seed_in;               /* first seed                               */

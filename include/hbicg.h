@@ -78,7 +78,18 @@ typedef struct hbicg_params {
                             within 16-bit column offsets of their tile (stencils), else
                             formed for every row first and gathered; 1: always at the
                             gathered columns; 2: always beforehand.  Same results.        */
-    int    fused;        /* default mode: 1 (default) four launches per iteration --
+    int    fused;        /* default mode: 1 (default), where the plan fits it (every
+                            256 rows hold at most 2048 entries, the matrix at most 16
+                            diagonals, columns ascending, n <= 2097152, window >= 16,
+                            no profile) the resident form: one launch runs many
+                            iterations, workgroups keeping their rows' vectors in
+                            registers and LDS, and one advances the shifts over
+                            them; should its workgroups not all become resident,
+                            the solve goes on in launches.  4: as 1, but a resident
+                            launch does not wait for its workgroups to become
+                            resident (a solve of more than one workgroup goes on in
+                            launches at once; for tests).
+                            Elsewhere four launches per iteration --
                             the alpha~ finalize runs as the first workgroup of SpMV
                             2's launch (where SpMV 2 forms q at its gathered columns
                             in one pass; else it keeps its own launch), the omega~
