@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 
+#include "hb_pool.h"
 #include "hb_shared.h"
 #include "../../include/hbicg.h"
 
@@ -279,8 +280,8 @@ extern "C" int hbicg_coo2csr_device(const unsigned *row, const unsigned *col, co
     const size_t scan_tmp = (hlen + SC_TILE - 1) / SC_TILE + 1;
     /* one allocation: flag, keys x2, positions x2, histogram, scan partials */
     const size_t words = 64 + (passes ? 4 * (size_t)nz + hlen + scan_tmp : 0);
-    unsigned *buf = nullptr;
-    if (hipMalloc((void **)&buf, words * sizeof(unsigned)) != hipSuccess) return HBICG_E_NOMEM;
+    unsigned *buf = (unsigned *)hb_pool_get(words * sizeof(unsigned));
+    if (!buf) return HBICG_E_NOMEM;
     int rc = 0;
     unsigned bad = 0;
     unsigned *flag = buf;
@@ -326,7 +327,7 @@ extern "C" int hbicg_coo2csr_device(const unsigned *row, const unsigned *col, co
     if (e != hipSuccess) rc = HBICG_E_HIP;
 done:
     (void)hipStreamSynchronize(s);
-    (void)hipFree(buf);
+    hb_pool_put(buf);
     return rc;
 }
 

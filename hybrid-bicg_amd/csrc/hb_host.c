@@ -20,6 +20,7 @@
 
 #include "hb_adjoint.h"
 #include "hb_launch.h"
+#include "hb_pool.h"
 #include "hb_shared.h"
 #include "../../include/hbicg.h"
 
@@ -179,12 +180,8 @@ static int build_blocks(const unsigned *ptr, int n, unsigned **out, int *nblk)
 
 static void *dalloc(size_t bytes, int *rc)
 {
-    void *p = NULL;
-    if (bytes == 0) bytes = 8;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        *rc = HBICG_E_NOMEM;
-        return NULL;
-    }
+    void *p = hb_pool_get(bytes);
+    if (!p) *rc = HBICG_E_NOMEM;
     return p;
 }
 
@@ -195,14 +192,14 @@ void hbicg_plan_destroy(hbicg_plan *pl)
     if (pl->stream) hipStreamSynchronize(pl->stream);
     if (pl->gexec) hipGraphExecDestroy(pl->gexec);
     if (pl->graph_obj) hipGraphDestroy(pl->graph_obj);
-    if (pl->own_matrix) { hipFree(pl->val); hipFree(pl->col); hipFree(pl->ptr); }
+    if (pl->own_matrix) { hb_pool_put(pl->val); hb_pool_put(pl->col); hb_pool_put(pl->ptr); }
     void *bufs[] = {pl->blk, pl->col16, pl->cflag, pl->rhat, pl->rring, pl->qring, pl->s, pl->y, pl->p_set, pl->x_host_buf,
                     pl->b_buf, pl->sigma, pl->aa, pl->ba, pl->wa, pl->pi, pl->eta, pl->zeta,
                     pl->coef, pl->ccoef, pl->grow, pl->part, pl->trace, pl->p_snap, pl->vidx, pl->vdict, pl->col16p, pl->tpad, pl->dtile, pl->doff, pl->didx, pl->dval, pl->pval, pl->pcol, pl->pptr, pl->pblk, pl->flush_log, pl->stop, pl->stop_iter, pl->act_len, pl->flist, pl->fpos,
                     pl->switch_k, pl->switch_to, pl->st, pl->rend, pl->rpres, pl->rdia,
                     pl->pring, pl->drlog, pl->qqlog, pl->mail};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
-        if (bufs[i]) hipFree(bufs[i]);
+        hb_pool_put(bufs[i]);
     if (pl->flag_host) hipHostFree(pl->flag_host);
     for (int i = 0; i < 2; ++i) if (pl->ev[i]) hipEventDestroy(pl->ev[i]);
     if (pl->t0) hipEventDestroy(pl->t0);
@@ -613,7 +610,7 @@ static int build_panels(hbicg_plan *pl, const hbicg_csr *A, int a_on_device, con
          * tiles any pass has, in each phase's slice */
         double *np = (double *)dalloc((size_t)grow * 6 * 8, &rc);
         if (rc) goto done;
-        hipFree(pl->part);
+        hb_pool_put(pl->part);
         pl->part = np;
         pl->maxparts = grow;
         pl->dev.part = np;
@@ -727,7 +724,8 @@ static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
     d->res_join = join;
     d->res_G = G;
 fail:
-    if (work) hipFree(work);
+    if (rc) hipStreamSynchronize(pl->stream);
+    hb_pool_put(work);
     free(host);
     return rc;
 }
@@ -764,6 +762,7 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
     {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+        else free_b += hb_pool_held();
         pl->W = window_for(p, variant, w_cap, (size_t)n, free_b);
     }
     pl->cap = p->max_iter + 1;
@@ -1413,8 +1412,9 @@ int hbicg_plan_true_residuals(hbicg_plan *pl, const double *b, const double *sig
     HIPCK(hipMemcpyAsync(out, dout, (size_t)pl->M * 8, hipMemcpyDeviceToHost, pl->stream));
     HIPCK(hipStreamSynchronize(pl->stream));
 fail:
-    if (part) hipFree(part);
-    if (dout) hipFree(dout);
+    if (rc) hipStreamSynchronize(pl->stream);
+    hb_pool_put(part);
+    hb_pool_put(dout);
     return rc;
 }
 
@@ -1562,21 +1562,21 @@ void hbicg_batch_destroy(hbicg_batch *bt)
         if (bt->gexec[l]) hipGraphExecDestroy(bt->gexec[l]);
         if (bt->graph_obj[l]) hipGraphDestroy(bt->graph_obj[l]);
     }
-    for (int ph = 0; ph < HB_NPH; ++ph) if (bt->a_tab[ph]) hipFree(bt->a_tab[ph]);
-    if (bt->act) hipFree(bt->act);
-    if (bt->pofs) hipFree(bt->pofs);
-    if (bt->pcnt) hipFree(bt->pcnt);
+    for (int ph = 0; ph < HB_NPH; ++ph) hb_pool_put(bt->a_tab[ph]);
+    hb_pool_put(bt->act);
+    hb_pool_put(bt->pofs);
+    hb_pool_put(bt->pcnt);
     free(bt->hpofs);
     free(bt->hpcnt);
     if (bt->plans)
         for (int p = 0; p < bt->nprob; ++p) hbicg_plan_destroy(bt->plans[p]);
     free(bt->plans);
     free(bt->hdevs);
-    if (bt->ddevs) hipFree(bt->ddevs);
-    if (bt->t_spmv) hipFree(bt->t_spmv);
-    if (bt->t_vec) hipFree(bt->t_vec);
-    if (bt->t_shift) hipFree(bt->t_shift);
-    if (bt->t_coef) hipFree(bt->t_coef);
+    hb_pool_put(bt->ddevs);
+    hb_pool_put(bt->t_spmv);
+    hb_pool_put(bt->t_vec);
+    hb_pool_put(bt->t_shift);
+    hb_pool_put(bt->t_coef);
     if (bt->flag_host) hipHostFree(bt->flag_host);
     for (int i = 0; i < 2; ++i) if (bt->ev[i]) hipEventDestroy(bt->ev[i]);
     if (bt->t0) hipEventDestroy(bt->t0);
@@ -1621,9 +1621,9 @@ static int batch_layout(hbicg_batch *bt, int W, int group_cap)
         const hb_dev *d = &bt->hdevs[p];
         for (int i = 0; i < d->shift_gx * d->shift_gy; ++i) { tab[2 * t] = p; tab[2 * t + 1] = i; ++t; }
     }
-    if (bt->t_shift) hipFree(bt->t_shift);
+    hb_pool_put(bt->t_shift);
     bt->t_shift = (int *)dalloc(tiles * 2 * sizeof(int), &rc);
-    if (bt->a_tab[HB_PH_SHIFT]) hipFree(bt->a_tab[HB_PH_SHIFT]);
+    hb_pool_put(bt->a_tab[HB_PH_SHIFT]);
     bt->a_tab[HB_PH_SHIFT] = (int *)dalloc(tiles * 2 * sizeof(int), &rc);
     if (rc) { free(tab); return rc; }
     HIPCK(hipMemcpy(bt->t_shift, tab, tiles * 2 * sizeof(int), hipMemcpyHostToDevice));
@@ -1685,6 +1685,7 @@ hbicg_batch *hbicg_batch_create(const hbicg_csr *A, int a_on_device, int nprob, 
         double rows = 0.0;
         for (int q = 0; q < nprob; ++q) rows += (double)A[q].n;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+        else free_b += hb_pool_held();
         while (wmax > 16 && (2.0 * wmax + 1.0) * rows * 8.0 > 0.25 * (double)free_b) wmax /= 2;
     }
     bt->wmax = wmax;
@@ -2013,7 +2014,8 @@ int hbicg_csr_transpose(const hbicg_csr *A, unsigned *tptr, unsigned *tcol, doub
     }
     HIPCK(hipStreamSynchronize(s));
 fail:
-    hipFree(work);
+    if (rc) hipStreamSynchronize(s);   /* nothing may still use it */
+    hb_pool_put(work);
     return rc;
 }
 
@@ -2033,7 +2035,8 @@ int hbicg_csr_transpose_pattern(const hbicg_csr *A, unsigned *tptr, unsigned *tc
     }
     HIPCK(hipStreamSynchronize(s));
 fail:
-    hipFree(work);
+    if (rc) hipStreamSynchronize(s);   /* nothing may still use it */
+    hb_pool_put(work);
     return rc;
 }
 
@@ -2075,7 +2078,8 @@ int hbicg_adjoint_gradients(const hbicg_csr *A, int M, const double *mu, const d
     if (rc) goto fail;
     HIPCK(hipStreamSynchronize(s));
 fail:
-    hipFree(work);
+    if (rc) hipStreamSynchronize(s);   /* nothing may still use it */
+    hb_pool_put(work);
     return rc;
 }
 

@@ -95,7 +95,7 @@ EXPORTS = {
                 "hbicg_batch_true_residuals", "hbicg_batch_autotune", "hbicg_csr_transpose",
                 "hbicg_csr_transpose_pattern", "hbicg_gather_values", "hbicg_adjoint_gradients",
                 "hbicg_adjoint_work_bytes", "hbicg_adjoint_gradients_ws", "hbicg_coo2csr_device", "hbicg_csr_load_device",
-                "hbicg_csr_free_device"],
+                "hbicg_csr_free_device", "hbicg_trim"],
 }
 
 _lib = None
@@ -204,6 +204,8 @@ def load():
     L.hbicg_csr_load_device.restype = C.c_int
     L.hbicg_csr_free_device.argtypes = [C.POINTER(Csr)]
     L.hbicg_csr_free_device.restype = None
+    L.hbicg_trim.argtypes = []
+    L.hbicg_trim.restype = None
     _lib = L
     return L
 

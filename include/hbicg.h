@@ -166,6 +166,10 @@ int  hbicg_last_residual_trace(double *out, int M, int rows);
 int  hbicg_last_report(hbicg_report *rep, int *stop_iter, int M,
                        int *switch_k, int *switch_to, int max_switch);
 
+/* Frees the device memory kept from destroyed plans for later ones (at most
+ * 1/32 of the device's memory; also freed when an allocation fails). */
+void hbicg_trim(void);
+
 /* ---- device-resident plan ------------------------------------------------ */
 typedef struct hbicg_csr {
     const double   *val;

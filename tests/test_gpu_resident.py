@@ -137,3 +137,29 @@ def test_values_in_place():
     fresh = Plan(None, 3, make_params(tol=1e-10, graph=1, value_index=False, fused=0), tensors=t)
     _, want, _ = fresh.solve(b, sig, 0)
     assert torch.equal(x, want)
+
+
+def test_memory_kept_between_plans():
+    """plans that follow each other run on the memory of those before, from
+    two threads too, and give the same results"""
+    import threading
+
+    from hbicg import _lib
+    A, B = P.conv_diff_2d(70, 60, 4.01), P.conv_diff_3d(25, 24, 23)
+    want = {id(A): _run(A, 6, 0, fused=0), id(B): _run(B, 6, 0, fused=0)}
+    got = []
+
+    def turns(order):
+        for M in order:
+            got.append((id(M), _run(M, 6, 0)))
+
+    ts = [threading.Thread(target=turns, args=(o,)) for o in ((A, B, A, B), (B, B, A, A))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    _lib.load().hbicg_trim()
+    turns((A, B))
+    assert len(got) == 10
+    for key, g in got:
+        _same(g, want[key])
