@@ -558,7 +558,19 @@ DEV void spmv_body(const hb_dev &d, unsigned b, const double *__restrict__ val,
                  * the row is summed in CSR order across the panels */
                 double acc = lane == 0 ? cin : 0.0;
                 const int hi = (int)rp[row + 1];
-                for (int e = (int)rp[row] + lane; e < hi; e += T) acc += prod[e];
+                int e = (int)rp[row] + lane;
+                /* a long row in a tile of many (power-law rows: two lanes for
+                 * hundreds of entries): eight reads in flight, added in order.
+                 * One read per addition took 45 us a SpMV on 60000 such rows,
+                 * most of it in the tiles that hold one */
+                for (; e + 7 * T < hi; e += 8 * T) {
+                    double v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = prod[e + u * T];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc += v[u];
+                }
+                for (; e < hi; e += T) acc += prod[e];
                 for (int o = T >> 1; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
                 if (lane == 0) finish(i_me, acc, oa, ob, oc);
             }
@@ -2329,34 +2341,77 @@ __global__ void k_publish(const hb_state *st, int *flag)
 }
 
 /* ---- true residual of every shift ----------------------------------------
- * out[j] = ||b - (A + sigma_j I) x_j|| / ||b|| in FP64: grid (R, M), the R
- * workgroups of shift j striding over the rows; row i's product summed in
- * CSR order, then + sigma_j x_i and - b_i as the reference forms it
- * (src/solver_dynamic.c:405-421, src/matrix.c:498-516); the squared entries
- * go to one partial pair per workgroup, combined in a fixed order per shift.
- * R depends only on (n, M), so every caller gets the same roundings. */
+ * out[j] = ||b - (A + sigma_j I) x_j|| / ||b|| in FP64: R workgroups for each
+ * group of HB_RJ shifts (workgroup r of group g is g + groups r) stride over the rows;
+ * row i's product is summed in CSR order, then + sigma_j x_i and - b_i as the
+ * reference forms it (src/solver_dynamic.c:405-421, src/matrix.c:498-516); the
+ * squared entries go to one partial pair per workgroup and shift, combined in
+ * a fixed order per shift.  R depends only on (n, M), so every caller gets
+ * the same roundings.  An entry of A is read once for the group, not once
+ * per shift, and the groups of the same rows run side by side. */
+#define HB_RJ 8
+
 __global__ __launch_bounds__(HB_BLOCK) void k_resid_part(hb_dev d, const double *__restrict__ b,
                                                          const double *__restrict__ sigma,
                                                          const double *__restrict__ x_set,
                                                          double *__restrict__ part)
 {
-    const int j = blockIdx.y;
-    const double *__restrict__ x = x_set + off(j, d.n);
-    const double sj = sigma[j];
-    double e2 = 0.0, b2 = 0.0;
-    for (int i = blockIdx.x * HB_BLOCK + threadIdx.x; i < d.n; i += gridDim.x * HB_BLOCK) {
-        double t = 0.0;
-        for (unsigned e = d.ptr[i]; e < d.ptr[i + 1]; ++e) t += d.val[e] * x[d.col[e]];
-        t = t + sj * x[i];
+    const int groups = (d.M + HB_RJ - 1) / HB_RJ, R = gridDim.x / groups, wg = blockIdx.x / groups;
+    const int j0 = (blockIdx.x % groups) * HB_RJ, nj = min(HB_RJ, d.M - j0), n = d.n;
+    const unsigned *__restrict__ ptr = d.ptr, *__restrict__ col = d.col;
+    const double *__restrict__ val = d.val;
+    /* shifts past the last repeat it: loaded, not stored */
+    size_t xo[HB_RJ];
+#pragma unroll
+    for (int u = 0; u < HB_RJ; ++u) xo[u] = off(j0 + min(u, nj - 1), n);
+    double e2[HB_RJ], b2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < HB_RJ; ++u) e2[u] = 0.0;
+    for (int i = wg * HB_BLOCK + threadIdx.x; i < n; i += R * HB_BLOCK) {
+        double t[HB_RJ];
+#pragma unroll
+        for (int u = 0; u < HB_RJ; ++u) t[u] = 0.0;
+        const unsigned e1 = ptr[i + 1];
+        for (unsigned e = ptr[i]; e < e1; e += 4) {
+            /* four entries' values, columns and gathers in flight */
+            double a[4];
+            unsigned c[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const unsigned f = min(e + q, e1 - 1);
+                a[q] = val[f];
+                c[q] = col[f];
+            }
+#pragma unroll
+            for (int u = 0; u < HB_RJ; ++u) {
+                const double *__restrict__ x = x_set + xo[u];
+                double xv[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xv[q] = x[c[q]];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double s = t[u] + a[q] * xv[q];
+                    t[u] = e + q < e1 ? s : t[u];
+                }
+            }
+        }
         const double bi = b[i];
-        const double e1 = t - bi;
-        e2 += e1 * e1;
+#pragma unroll
+        for (int u = 0; u < HB_RJ; ++u) {
+            const double r = t[u] + sigma[j0 + min(u, nj - 1)] * x_set[xo[u] + i];
+            const double e1 = r - bi;
+            e2[u] += e1 * e1;
+        }
         b2 += bi * bi;
     }
-    block_sum2(e2, b2);
-    if (threadIdx.x == 0) {
-        part[((size_t)j * gridDim.x + blockIdx.x) * 2] = e2;
-        part[((size_t)j * gridDim.x + blockIdx.x) * 2 + 1] = b2;
+#pragma unroll
+    for (int u = 0; u < HB_RJ; ++u) {
+        double e = e2[u], s2 = b2;
+        block_sum2(e, s2);
+        if (threadIdx.x == 0 && u < nj) {
+            part[((size_t)(j0 + u) * R + wg) * 2] = e;
+            part[((size_t)(j0 + u) * R + wg) * 2 + 1] = s2;
+        }
     }
 }
 
@@ -2797,7 +2852,7 @@ int hb_k_true_residual(const hb_dev *d, const double *b, const double *sigma, co
                        double *part, double *out, hipStream_t s)
 {
     const int R = hb_k_resid_blocks(d->n, d->M);
-    hipLaunchKernelGGL(k_resid_part, dim3(R, d->M), dim3(HB_BLOCK), 0, s, *d, b, sigma, x, part);
+    hipLaunchKernelGGL(k_resid_part, dim3((d->M + HB_RJ - 1) / HB_RJ * R), dim3(HB_BLOCK), 0, s, *d, b, sigma, x, part);
     hipLaunchKernelGGL(k_resid_final, dim3(d->M), dim3(HB_BLOCK), 0, s, part, R, out);
     return (int)hipGetLastError();
 }
