@@ -39,7 +39,6 @@
  * (src/openmp_vector.c:68-74, src/openmp_matrix.c:47-58).
  */
 #include <hip/hip_runtime.h>
-#include <type_traits>
 #include <math.h>
 #include "hb_shared.h"
 #include "hb_launch.h"
@@ -2075,7 +2074,7 @@ DEV dbl2 p_step2(dbl2 p, dbl2 r, dbl2 s, double pb, double pbw)
  * their loads run while the stage does.  Then, when the stage has decided a
  * flush and the combined coefficients are in, the workgroup applies flush
  * tiles t, t + T, ...  The solve's last flush (x_j only, the longest) is left
- * to k_flush_final after the loop: in this kernel the compiler keeps one of
+ * to k_flush_mm after the loop: in this kernel the compiler keeps one of
  * a window step's four coefficient blocks in flight instead of four, and
  * that flush ran 6.9 ms here against 4.3 ms in a kernel of its own. */
 DEV void shift_stage_tiles(const hb_dev &d, int t, int T)
@@ -2167,31 +2166,197 @@ DEV void shift_stage_tiles(const hb_dev &d, int t, int T)
     }
 }
 
-/* The solve's last window flush (x_j only) after the iteration loop, when the
- * shift kernel runs the scalar stage (or in the resident form): that iteration's stage marked it
- * (flush, flush_xonly) and its coefficient workgroups formed the combined
- * coefficients.  One workgroup per 256-element tile. */
-__global__ __launch_bounds__(HB_BLOCK) void k_flush_final(hb_dev d)
+/* The window flush on the matrix cores.  Per 16 list positions (a chunk) and
+ * 16 elements it is a product of the chunk's coefficients with the window's
+ * vectors, accumulated onto x_j (and p_j): v_mfma_f64_16x16x4 takes four
+ * vectors a step and adds their products in ascending order with fused
+ * multiply-adds, so the results are bitwise those of flush_apply and
+ * flush_apply_x2.  Lane l holds coefficient row l / 16 of the step for
+ * position l % 16, the same vector's element l % 16, and of the result
+ * positions l / 16 + 4 r, element l % 16.
+ *
+ * A wave takes MB chunks and 16 NB elements: an element of a window vector
+ * is loaded once for up to 64 shifts, where the vector form loads it once per
+ * 16 shifts and 64 lanes and waits for scalar coefficient loads in every
+ * step.  The next step's operands are loaded ahead of a step's products.
+ * Bound: the vectors' traffic up to about 64 shifts and the FP64 rate beyond
+ * (128^3, 318 iterations, 64 shifts: 11.7 GB, 2.3 ms at a copy's rate, and
+ * 0.17 TFLOP, 2.4 ms at a large product's).  Against the vector form in a
+ * launch of its own: that flush 3.68 -> 3.44 ms; 512 shifts at 64^3, x_j and
+ * p_j 4.18 -> 2.55 ms; 23 shifts at 251 x 173, 643 -> 93 us; 16 at 64 x 64,
+ * 209 -> 16 us. */
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+template <int MB, int NB, bool XONLY>
+DEV void flush_mm(const hb_dev &d, int eb, int sg, const hb_fl &fw, int snap_k)
 {
-    const hb_state *st = d.st;
-    if (!st->flush || !st->flush_xonly) return;
-    const hb_fl fw = flush_window(st->flush_k0, st->flush_cnt, st->flush_len, st->flush_tail, st->win_seedpos);
-    flush_apply_x2<HB_UG>(d, blockIdx.x, fw, d.x_set, d.p_set, d.rring, d.qring, d.ccoef, d.flist);
+    const int n = d.n, W = d.W, k0 = fw.k0, cnt = fw.cnt, Lc = fw.Lc, tail = XONLY ? 0 : fw.tail;
+    const int lane = threadIdx.x & 63, c16 = lane & 15, kq = lane >> 4;
+    const int nch = (cnt + HB_UG - 1) / HB_UG, ch0 = sg * MB;
+    if (ch0 >= nch || eb * (16 * NB) >= n) return;
+    const size_t cstride = (size_t)HB_CC_ROWS(W) * (2 * HB_UG);
+    const double *cc = d.ccoef + (size_t)ch0 * cstride;
+    int i[NB];
+    bool in[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int e = eb * (16 * NB) + 16 * b + c16;
+        in[b] = e < n;
+        i[b] = in[b] ? e : n - 1;
+    }
+    /* coefficient rows of each chunk: a chunk ends at the latest step any of
+     * its shifts was updated in (rows of stopped shifts are zero) */
+    int K[MB], Kmax = 0;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const int pos = (ch0 + m) * HB_UG + c16;
+        int nb = pos < cnt ? min(d.act_len[pos], Lc) : -1;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) nb = max(nb, __shfl_xor(nb, o, 64));
+        nb = __builtin_amdgcn_readfirstlane(nb);
+        K[m] = nb < 0 ? 0 : 2 * (tail ? Lc : nb) + 1;
+        Kmax = max(Kmax, K[m]);
+    }
+    dbl4 x[MB][NB], p[XONLY ? 1 : MB][NB];
+    const bool first = k0 == 1, xz = first && d.x_zero;
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int u = kq + 4 * r, pos = (ch0 + m) * HB_UG + u;
+            const bool has = pos < cnt;
+            const int j = d.flist[has ? pos : 0];
+            const double *cb = cc + (K[m] ? m * cstride : 0);
+            const double cx = cb[u], cp = cb[HB_UG + u];
+            /* the first window starts from p_j = b for every shift; the seed's
+             * window-start p is the snapshot */
+            const double *ps = first ? (const double *)d.b_in : pos == fw.sp ? (const double *)d.p_snap
+                                                                             : (const double *)d.p_set + off(j, n);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const double p0 = ps[i[b]];
+                const double x0 = xz ? 0.0 : __builtin_nontemporal_load((const double *)d.x_set + off(j, n) + i[b]);
+                x[m][b][r] = __builtin_fma(cx, p0, x0);
+                if (!XONLY) p[XONLY ? 0 : m][b][r] = cp * p0;
+            }
+        }
+    /* lane's vectors k = kq, kq + 4, ...: r_{k0-1+k/2} for even k,
+     * q_{k0+(k-1)/2} for odd */
+    const bool odd = kq & 1;
+    const int mod = odd ? W : W + 1;
+    const double *ring = odd ? (const double *)d.qring : (const double *)d.rring;
+    int slot = (odd ? k0 + (kq >> 1) : k0 - 1 + (kq >> 1)) % mod;
+    int k = kq;
+    auto load = [&](double (&a)[MB], double (&ap)[MB], double (&g)[NB]) {
+        const bool on = k < Kmax;
+        const double *v = ring + off(slot, n);
+        const int row = 1 + min(k, Kmax - 1);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) g[b] = v[i[b]];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            const double *cr = cc + (K[m] ? m * cstride : 0) + row * (2 * HB_UG) + c16;
+            a[m] = cr[0];
+            ap[m] = XONLY ? 0.0 : cr[HB_UG];
+        }
+        /* past the end: rows of an earlier window, slots not written yet */
+#pragma unroll
+        for (int b = 0; b < NB; ++b) g[b] = on ? g[b] : 0.0;
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            a[m] = on ? a[m] : 0.0;
+            ap[m] = on ? ap[m] : 0.0;
+        }
+        k += 4;
+        slot += 2;
+        while (slot >= mod) slot -= mod;
+    };
+    auto step = [&](int s, const double (&a)[MB], const double (&ap)[MB], const double (&g)[NB]) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            if (4 * s >= K[m]) continue;   /* uniform */
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                x[m][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], g[b], x[m][b], 0, 0, 0);
+                if (!XONLY)
+                    p[XONLY ? 0 : m][b] =
+                        __builtin_amdgcn_mfma_f64_16x16x4f64(ap[m], g[b], p[XONLY ? 0 : m][b], 0, 0, 0);
+            }
+        }
+    };
+    const int steps = (Kmax + 3) / 4;
+    double a0[MB], p0[MB], g0[NB], a1[MB], p1[MB], g1[NB];
+    load(a0, p0, g0);
+    for (int s = 0; s < steps; s += 2) {
+        load(a1, p1, g1);
+        step(s, a0, p0, g0);
+        load(a0, p0, g0);
+        step(s + 1, a1, p1, g1);
+    }
+    if (tail) {
+        /* the window's last iteration on its own (src/solver_dynamic.c:248-255) */
+        const double *gq = d.qring + off((k0 + Lc) % W, n), *gr = d.rring + off((k0 + Lc - 1) % (W + 1), n);
+        const double *gn = d.rring + off((k0 + Lc) % (W + 1), n);
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double *ct = cc + (K[m] ? m * cstride : 0) + (size_t)(2 * W + 2) * (2 * HB_UG) + kq + 4 * r;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const double q = gq[i[b]];
+                    const int mp = XONLY ? 0 : m;
+                    double xe = __builtin_fma(ct[0], q, x[m][b][r]);
+                    xe = __builtin_fma(ct[HB_UG], p[mp][b][r], xe);
+                    double pe = __builtin_fma(ct[2 * HB_UG], q, p[mp][b][r]);
+                    pe = __builtin_fma(ct[3 * HB_UG], gr[i[b]], pe);
+                    pe = ct[4 * HB_UG] * pe;
+                    p[mp][b][r] = __builtin_fma(ct[5 * HB_UG], gn[i[b]], pe);
+                    x[m][b][r] = xe;
+                }
+            }
+    }
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int pos = (ch0 + m) * HB_UG + kq + 4 * r;
+            if (pos >= cnt) continue;
+            const int j = d.flist[pos];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if (!in[b]) continue;
+                __builtin_nontemporal_store(x[m][b][r], (double *)d.x_set + off(j, n) + i[b]);
+                /* the seed keeps its own p (the regrouped one is only its x's
+                 * companion) */
+                if (!XONLY && pos != fw.sp)
+                    __builtin_nontemporal_store(p[XONLY ? 0 : m][b][r], (double *)d.p_set + off(j, n) + i[b]);
+            }
+        }
+    /* the resident form's next window has begun already: its snapshot, by the
+     * wave that read the old one above (the seed's chunk) */
+    if (!XONLY && snap_k && sg == max(fw.sp, 0) / (HB_UG * MB) && kq == 0) {
+        const double *ps = d.pring + off(snap_k % d.res_P, n);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            if (in[b]) d.p_snap[i[b]] = ps[i[b]];
+    }
 }
 
-/* A window flush of the resident form that is not the solve's last. */
-__global__ __launch_bounds__(HB_BLOCK) void k_res_flush(hb_dev d)
+/* FINAL: the solve's last flush (x_j only), after the iteration loop, when
+ * the shift kernel runs the scalar stage or in the resident form; else a
+ * flush of the resident form between launches.  The groups of MB chunks of
+ * the same elements run side by side on one XCD. */
+template <int MB, int NB, bool FINAL>
+__global__ __launch_bounds__(HB_BLOCK, MB * NB * (FINAL ? 1 : 2) >= 8 ? 3 : 4) void k_flush_mm(hb_dev d, int groups)
 {
     const hb_state *st = d.st;
-    if (st->res_flush != 1) return;
+    if (FINAL ? !st->flush || !st->flush_xonly : st->res_flush != 1) return;
     const hb_fl fw = flush_window(st->flush_k0, st->flush_cnt, st->flush_len, st->flush_tail, st->win_seedpos);
-    flush_apply<HB_UG>(d, blockIdx.x, fw, d.x_set, d.p_set, d.rring, d.qring, d.ccoef, d.flist);
-    const int ks = st->res_snap;
-    if (ks) {
-        __syncthreads();   /* the tile's old snapshot has been read */
-        const int i = blockIdx.x * HB_BLOCK + threadIdx.x;
-        if (i < d.n) d.p_snap[i] = d.pring[off(ks % d.res_P, d.n) + i];
-    }
+    const unsigned wg = xcd_tile(blockIdx.x, gridDim.x);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    flush_mm<MB, NB, FINAL>(d, (int)(wg / groups) * (HB_BLOCK / 64) + wave, (int)(wg % groups), fw,
+                            FINAL ? 0 : st->res_snap);
 }
 
 /* Shift kernel with the scalar stage (default mode, fused level 1):
@@ -2618,6 +2783,36 @@ static void spmv_panels(const hb_dev *d, hipStream_t s)
                        P - 1);
 }
 
+template <int MB, int NB, bool FINAL>
+static void launch_flush_as(const hb_dev *d, hipStream_t s)
+{
+    const int chunks = (d->M + HB_UG - 1) / HB_UG, groups = (chunks + MB - 1) / MB, ne = HB_BLOCK / 64 * 16 * NB;
+    hipLaunchKernelGGL((k_flush_mm<MB, NB, FINAL>), dim3((unsigned)((d->n + ne - 1) / ne * groups)), dim3(HB_BLOCK), 0,
+                       s, *d, groups);
+}
+
+/* Chunks and elements per wave.  A flush that is not the last: up to two
+ * chunks (x_j and p_j take the registers of four) and 32 elements.  The last
+ * one: four chunks and 32 elements where that is one wave's whole list, so
+ * that each vector is read once (33 to 64 shifts at 128^3: 3.44 ms, against
+ * 4.00 with two chunks and 64 elements and 4.22 with two and 32); else two
+ * chunks and 64 elements, whose stores of x_j are 512 bytes to a row (32
+ * shifts at 112^3: 1.42 ms against 1.52 with 32 elements; 512 shifts at
+ * 64^3: 1.42 against 1.63 with four chunks and 32).  Fewer elements where
+ * the grid would leave fewer than two waves per SIMD of the 1024 to hide the
+ * loads' latency. */
+template <bool FINAL>
+static void launch_flush(const hb_dev *d, hipStream_t s)
+{
+    const int chunks = (d->M + HB_UG - 1) / HB_UG;
+    auto fits = [&](int mb, int ne) { return (size_t)d->n / ne * ((chunks + mb - 1) / mb) >= 2048; };
+    if (chunks == 1) fits(1, 32) ? launch_flush_as<1, 2, FINAL>(d, s) : launch_flush_as<1, 1, FINAL>(d, s);
+    else if (!FINAL) fits(2, 32) ? launch_flush_as<2, 2, false>(d, s) : launch_flush_as<2, 1, false>(d, s);
+    else if ((chunks == 3 || chunks == 4) && fits(4, 32)) launch_flush_as<4, 2, true>(d, s);
+    else if (chunks != 3 && chunks != 4 && fits(2, 64)) launch_flush_as<2, 4, true>(d, s);
+    else fits(2, 32) ? launch_flush_as<2, 2, true>(d, s) : launch_flush_as<2, 1, true>(d, s);
+}
+
 template <int WM, int V, int U>
 static void launch_shift(const hb_dev *d, hipStream_t s)
 {
@@ -2829,7 +3024,7 @@ int hb_k_publish(const hb_dev *d, int *flag_dev, hipStream_t s)
 
 int hb_k_finalize(const hb_dev *d, hipStream_t s)
 {
-    if (d->fused_s || d->res_G) hipLaunchKernelGGL(k_flush_final, dim3(d->shift_gx), dim3(HB_BLOCK), 0, s, *d);
+    if (d->fused_s || d->res_G) launch_flush<true>(d, s);
     hipLaunchKernelGGL(k_finalize, dim3(d->vec_grid), dim3(HB_BLOCK), 0, s, *d);
     return (int)hipGetLastError();
 }
@@ -2837,7 +3032,7 @@ int hb_k_finalize(const hb_dev *d, hipStream_t s)
 int hb_k_res_flush(const hb_dev *d, hipStream_t s)
 {
     hipLaunchKernelGGL(k_res_coef, dim3(d->M, (2 * d->W + 2 + HB_BLOCK - 1) / HB_BLOCK), dim3(HB_BLOCK), 0, s, *d);
-    hipLaunchKernelGGL(k_res_flush, dim3(d->shift_gx), dim3(HB_BLOCK), 0, s, *d);
+    launch_flush<false>(d, s);
     return (int)hipGetLastError();
 }
 

@@ -112,6 +112,18 @@ def test_many_shifts():
     _same(_run(A, 1100, 900), _run(A, 1100, 900, fused=0))
 
 
+@pytest.mark.parametrize("x_zero", [True, False])
+@pytest.mark.parametrize("n", [7, 16, 33, 1000, 4096 + 65, 43700 + 1, 65536 + 17, 131072 + 63])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
+def test_flush_chunks(M, n, x_zero):
+    """The flush on the matrix cores (16 shifts a chunk, 16 to 64 elements a
+    wave) against the vector flush of the launches: a last chunk of one or 16
+    shifts, and the sizes around which the shapes of its waves change."""
+    A = _banded(n, [-2, 0, 1], 5, "const")
+    kw = dict(window=6, growth_limit=30.0, x_zero=x_zero)
+    _same(_run(A, M, 0, fused=1, **kw), _run(A, M, 0, fused=0, **kw))
+
+
 @pytest.mark.parametrize("M", [7, 300])
 @pytest.mark.parametrize("seed", [0, 5])
 def test_hand_over(M, seed):
