@@ -639,6 +639,14 @@ done:
     return rc;
 }
 
+static void free_resident(hbicg_plan *pl)
+{
+    hb_pool_put(pl->rpres); hb_pool_put(pl->rend); hb_pool_put(pl->pring); hb_pool_put(pl->drlog);
+    hb_pool_put(pl->qqlog); hb_pool_put(pl->mail); hb_pool_put(pl->rdia);
+    pl->rpres = NULL; pl->rend = NULL; pl->pring = NULL; pl->drlog = NULL;
+    pl->qqlog = NULL; pl->mail = NULL; pl->rdia = NULL;
+}
+
 /* The resident form of the default order (hb_resident.hip), where it fits:
  * every SpMV tile is 256 rows (at most 8 entries a row on average), the
  * matrix has at most HB_DIAG_K diagonals, columns ascending, and the rows fit
@@ -646,7 +654,7 @@ done:
  * launch-per-phase kernels.  A launch runs at most res_C iterations, whose
  * p stay in a ring (256 MiB of it, 32 slots at least): a window the growth
  * guard closes in the middle needs the p of its successor's first iteration. */
-static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
+static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join, int batched)
 {
     int rc = 0, cus = 0, SB = 0, E = 0, lcw = 0, bad = 0, K = 0;
     int *work = NULL, *host = NULL;
@@ -656,7 +664,8 @@ static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
     for (int t = 0; t < nblk; ++t)
         if (hblk[t] != (unsigned)t * HB_BLOCK) return 0;
     HIPCK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device));
-    const int G = hb_k_res_shape(nblk, cus, &SB, &E, &lcw);
+    /* a batch chooses its problems' shapes together (batch_resident) */
+    const int G = batched ? (hb_k_res_shape_b(nblk, 4, &lcw) ? 256 : 0) : hb_k_res_shape(nblk, cus, &SB, &E, &lcw);
     if (G <= 0) return 0;
     /* tile diagonals | their number | bad; then the value patterns */
     const size_t words = (size_t)nblk * (HB_DIAG_K + 1) + 1;
@@ -683,7 +692,7 @@ static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
             ++K;
         }
     if (K < 1) goto fail;
-    int KT = K <= 8 ? 8 : HB_DIAG_K;
+    int KT = K <= 8 && !batched ? 8 : HB_DIAG_K;
     if ((K == 5 || K == 7) && off[K / 2] == 0) KT = K;
     pl->rpres = (unsigned short *)dalloc((size_t)n * 2, &rc);
     if (rc) goto fail;
@@ -725,6 +734,11 @@ static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join)
     d->res_G = G;
 fail:
     if (rc) hipStreamSynchronize(pl->stream);
+    if (rc == HBICG_E_NOMEM) {
+        /* no room for it: the plan runs the launch-per-phase kernels */
+        free_resident(pl);
+        rc = 0;
+    }
     hb_pool_put(work);
     free(host);
     return rc;
@@ -963,8 +977,8 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
     }
     /* the resident form: default launches, windows long enough for a launch
      * to run a useful number of iterations */
-    if (d->fused && (p->fused == 1 || p->fused == 4) && !pl->profile && d->npanel <= 1 && pl->W >= HB_RES_WMIN &&
-        (rc = setup_resident(pl, hblk, p->fused == 4 ? 0 : HB_RES_JOIN)) != 0)
+    if (!pl->exact && (p->fused == 1 || p->fused == 4) && !pl->profile && d->npanel <= 1 && pl->W >= HB_RES_WMIN &&
+        (rc = setup_resident(pl, hblk, p->fused == 4 ? 0 : HB_RES_JOIN, batched)) != 0)
         goto fail;
     if (a_on_device) free(hptr);
     free(hblk);
@@ -1544,11 +1558,14 @@ struct hbicg_batch {
     int *hpofs, *hpcnt;        /* host [HB_NPH][nprob]: each problem's range in the full tables */
     int *pofs, *pcnt;          /* device copies                          */
     hb_batch B;
-    int *flag_host;            /* pinned: done, problems running, active entries per phase */
+    int *t_res;                /* the resident form's clusters (NULL: not used) */
+    int *flag_host;            /* pinned: done, problems running, active entries per phase,
+                                  problems the resident form has work for */
     hipEvent_t ev[2], t0, t1;
     hipGraphExec_t gexec[HB_GLEVELS];
     hipGraph_t graph_obj[HB_GLEVELS];
     int graph_dirty;
+    int res_full;              /* a problem's values are laid out at every solve */
     int levels_used;           /* bit l: the last run launched level l */
     double last_ms;
 };
@@ -1577,6 +1594,7 @@ void hbicg_batch_destroy(hbicg_batch *bt)
     hb_pool_put(bt->t_vec);
     hb_pool_put(bt->t_shift);
     hb_pool_put(bt->t_coef);
+    hb_pool_put(bt->t_res);
     if (bt->flag_host) hipHostFree(bt->flag_host);
     for (int i = 0; i < 2; ++i) if (bt->ev[i]) hipEventDestroy(bt->ev[i]);
     if (bt->t0) hipEventDestroy(bt->t0);
@@ -1649,6 +1667,67 @@ static int batch_layout(hbicg_batch *bt, int W, int group_cap)
 fail:
     free(tab);
     return rc;
+}
+
+/* The resident form for a batch: every problem or none (beside the
+ * launch-per-phase iterations of another problem, the rounds would add to the
+ * time of the batch).  A workgroup takes as few tiles as leave every cluster
+ * a compute unit per workgroup, 16 at most; the largest clusters first, so
+ * that those which must wait for compute units are the smallest. */
+static int batch_resident(hbicg_batch *bt)
+{
+    int rc = 0, cus = 0, SB, total = 0, *tab = NULL, *G = NULL, *lcw = NULL;
+    for (int q = 0; q < bt->nprob; ++q)
+        if (!bt->plans[q]->dev.res_G) goto none;
+    HIPCK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, bt->device));
+    G = (int *)malloc((size_t)bt->nprob * sizeof(int));
+    lcw = (int *)malloc((size_t)bt->nprob * sizeof(int));
+    if (!G || !lcw) { rc = HBICG_E_NOMEM; goto fail; }
+    for (SB = 1;; SB *= 2) {
+        int fits = 1;
+        total = 0;
+        for (int q = 0; q < bt->nprob; ++q) {
+            G[q] = hb_k_res_shape_b(bt->plans[q]->nblk, SB, &lcw[q]);
+            if (G[q] <= 0 || G[q] > cus) fits = 0;
+            total += G[q];
+        }
+        if (fits && (total <= cus || SB == 4)) break;
+        if (SB == 4) goto none;
+    }
+    tab = (int *)malloc((size_t)total * 2 * sizeof(int));
+    if (!tab) { rc = HBICG_E_NOMEM; goto fail; }
+    bt->t_res = (int *)dalloc((size_t)total * 2 * sizeof(int), &rc);
+    if (rc) goto fail;
+    int t = 0;
+    for (int g = 256; g > 0; --g)
+        for (int q = 0; q < bt->nprob; ++q) {
+            if (G[q] != g) continue;
+            for (int w = 0; w < g; ++w) { tab[2 * t] = q; tab[2 * t + 1] = w; ++t; }
+        }
+    HIPCK(hipMemcpy(bt->t_res, tab, (size_t)total * 2 * sizeof(int), hipMemcpyHostToDevice));
+    for (int q = 0; q < bt->nprob; ++q) {
+        hb_dev *d = &bt->hdevs[q];
+        d->res_G = G[q];
+        d->res_lcw = lcw[q];
+        d->res_SB = SB;
+        d->res_E = 1;
+        if (d->res_full) bt->res_full = 1;
+    }
+    bt->B.t_res = bt->t_res;
+    bt->B.n_res = total;
+    bt->B.res_SB = SB;
+    free(tab); free(G); free(lcw);
+    return 0;
+fail:
+    free(tab); free(G); free(lcw);
+    return rc;
+none:
+    free(G); free(lcw);
+    for (int q = 0; q < bt->nprob; ++q) {
+        bt->hdevs[q].res_G = bt->plans[q]->dev.res_G = 0;
+        free_resident(bt->plans[q]);
+    }
+    return 0;
 }
 
 hbicg_batch *hbicg_batch_create(const hbicg_csr *A, int a_on_device, int nprob, const int *M,
@@ -1759,7 +1838,7 @@ hbicg_batch *hbicg_batch_create(const hbicg_csr *A, int a_on_device, int nprob, 
     bt->B.pofs = bt->pofs;
     bt->B.pcnt = bt->pcnt;
     bt->B.div = 1;
-    HIPCK(hipHostMalloc((void **)&bt->flag_host, (2 + HB_NPH) * sizeof(int), hipHostMallocDefault));
+    HIPCK(hipHostMalloc((void **)&bt->flag_host, (3 + HB_NPH) * sizeof(int), hipHostMallocDefault));
     HIPCK(hipEventCreateWithFlags(&bt->ev[0], hipEventDisableTiming));
     HIPCK(hipEventCreateWithFlags(&bt->ev[1], hipEventDisableTiming));
     HIPCK(hipEventCreate(&bt->t0));
@@ -1778,6 +1857,7 @@ hbicg_batch *hbicg_batch_create(const hbicg_csr *A, int a_on_device, int nprob, 
     bt->B.n_vec_tiles = (int)nvec;
     bt->B.t_coef = bt->t_coef;
     bt->B.n_coef_tiles = (int)ncoef;
+    if ((rc = batch_resident(bt)) != 0) goto fail;
     {
         const int wdef = bt->exact || wmax < HB_WBATCH_DEF ? wmax : HB_WBATCH_DEF;
         if ((rc = batch_layout(bt, p->window > 0 && p->window < wmax ? p->window : wdef, 0)) != 0)
@@ -1840,6 +1920,33 @@ static int batch_level(const hbicg_batch *bt, int active_spmv)
     return l;
 }
 
+/* Rounds of the resident form (run_resident, for every problem at once): the
+ * host reads a round's flags while the next one runs. */
+static int batch_run_resident(hbicg_batch *bt, int max_cap)
+{
+    int rc = 0, launched = 0, prev = -1;
+    bt->flag_host[2 + HB_NPH] = bt->nprob;
+    if (bt->res_full && hb_kb_res_fill(&bt->B, bt->stream) != 0) return HBICG_E_HIP;
+    while (launched <= 2 * max_cap + 8) {
+        if (hb_kb_res_iterations(&bt->B, bt->stream) != 0 || hb_kb_res_flush(&bt->B, bt->stream) != 0 ||
+            hb_kb_publish(&bt->B, bt->flag_host, bt->stream) != 0)
+            return HBICG_E_HIP;
+        const int cur = launched & 1;
+        HIPCK(hipEventRecord(bt->ev[cur], bt->stream));
+        ++launched;
+        if (prev >= 0) {
+            HIPCK(hipEventSynchronize(bt->ev[prev]));
+            if (!__atomic_load_n(&bt->flag_host[2 + HB_NPH], __ATOMIC_ACQUIRE)) break;
+        }
+        prev = cur;
+    }
+    HIPCK(hipStreamSynchronize(bt->stream));
+    if (bt->flag_host[0]) return 0;
+    return hb_kb_res_leave(&bt->B, bt->stream) != 0 ? HBICG_E_HIP : 0;
+fail:
+    return rc;
+}
+
 /* Runs the batch with the current layout, max_iter_override > 0 capping
  * every problem's iterations (tuning runs).  b, x: per-problem pointers,
  * device memory; sigma: host arrays. */
@@ -1868,9 +1975,11 @@ static int batch_run(hbicg_batch *bt, const double *const *b, const double *cons
     if (hb_kb_init(&bt->B, bt->stream) != 0) return HBICG_E_HIP;
     bt->flag_host[0] = 0;
     bt->levels_used = 0;
+    /* windows long enough for a round to be worth its launches, as a plan's */
+    if (bt->t_res && bt->W >= HB_RES_WMIN && (rc = batch_run_resident(bt, max_cap)) != 0) return rc;
     const int max_chunks = max_cap / bt->chunk + 3;
     int launched = 0, prev = -1, level = 0;
-    for (;;) {
+    while (!bt->flag_host[0]) {
         bt->levels_used |= 1 << level;
         if (bt->graph) {
             if ((rc = batch_capture(bt, level)) != 0) return rc;

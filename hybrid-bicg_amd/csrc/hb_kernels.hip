@@ -1648,10 +1648,10 @@ __global__ __launch_bounds__(HB_BLOCK) void k_flush_coef(hb_dev d)
  * window's steps walked together by the workgroup so that a step's six
  * coefficients are uniform reads.  A component's walk starts where it first
  * is not zero; lanes before that keep their zeros. */
-__global__ __launch_bounds__(HB_BLOCK) void k_res_coef(hb_dev d)
+template <class D>
+DEV void res_coef_body(const D &d, int pos)
 {
     const hb_state *st = d.st;
-    const int pos = blockIdx.x;
     if (!st->res_flush || pos >= st->flush_cnt) return;
     const int M = d.M, W = d.W, L = st->flush_len, ntail = st->flush_tail;
     const int Lc = L - ntail, lv = d.act_len[pos], nb = min(lv, Lc);
@@ -1692,6 +1692,8 @@ __global__ __launch_bounds__(HB_BLOCK) void k_res_coef(hb_dev d)
         blk[(size_t)row * (2 * HB_UG) + HB_UG + pos % HB_UG] = pk.hi + pk.lo;
     }
 }
+
+__global__ __launch_bounds__(HB_BLOCK) void k_res_coef(hb_dev d) { res_coef_body(d, blockIdx.x); }
 
 /* The window a flush applies: its first iteration, list length, regrouped
  * iterations, tail flag and the seed's list position, uniform across the
@@ -2187,8 +2189,8 @@ DEV void shift_stage_tiles(const hb_dev &d, int t, int T)
  * 209 -> 16 us. */
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
-template <int MB, int NB, bool XONLY>
-DEV void flush_mm(const hb_dev &d, int eb, int sg, const hb_fl &fw, int snap_k)
+template <int MB, int NB, bool XONLY, class D>
+DEV void flush_mm(const D &d, int eb, int sg, const hb_fl &fw, int snap_k)
 {
     const int n = d.n, W = d.W, k0 = fw.k0, cnt = fw.cnt, Lc = fw.Lc, tail = XONLY ? 0 : fw.tail;
     const int lane = threadIdx.x & 63, c16 = lane & 15, kq = lane >> 4;
@@ -2662,6 +2664,43 @@ __global__ __launch_bounds__(HB_BLOCK) void kb_shift_cc(const hb_dev *__restrict
     for (int t = blockIdx.x; t < nt; t += gridDim.x) shift_cc_tile(devs[tab[2 * t]], tab[2 * t + 1]);
 }
 
+/* the resident form's rounds: tab as kb_flush_coef and kb_shift_cc */
+__global__ __launch_bounds__(HB_BLOCK) void kb_res_coef(const hb_dev *__restrict__ devs, const int *__restrict__ tab)
+{
+    const HB_K int *t = read_only(tab) + 2 * blockIdx.x;
+    res_coef_body(read_only(devs)[t[0]], t[1]);
+}
+
+/* 256 elements: each wave takes 64, 32 at a time through every chunk of the
+ * list.  The problem's last flush (x_j only) runs here too. */
+template <bool XONLY>
+DEV void res_flush_tile(const HB_K hb_dev &d, int tile, const hb_fl &fw, int snap_k)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int chunks = (fw.cnt + HB_UG - 1) / HB_UG;
+    for (int h = 0; h < 2; ++h) {
+        const int eb = tile * (HB_BLOCK / 32) + 2 * wave + h;
+        if (chunks == 1) {
+            flush_mm<1, 2, XONLY>(d, eb, 0, fw, snap_k);
+        } else {
+            for (int sg = 0; 2 * sg < chunks; ++sg) flush_mm<2, 2, XONLY>(d, eb, sg, fw, snap_k);
+        }
+    }
+}
+
+__global__ __launch_bounds__(HB_BLOCK, 4) void kb_res_flush(const hb_dev *__restrict__ devs,
+                                                            const int *__restrict__ tab)
+{
+    const HB_K int *t = read_only(tab) + 2 * blockIdx.x;
+    const HB_K hb_dev &d = read_only(devs)[t[0]];
+    const hb_state *st = d.st;
+    const int f = st->res_flush;
+    if (!f) return;
+    const hb_fl fw = flush_window(st->flush_k0, st->flush_cnt, st->flush_len, st->flush_tail, st->win_seedpos);
+    if (f == 2) res_flush_tile<true>(d, t[1], fw, 0);
+    else res_flush_tile<false>(d, t[1], fw, st->res_snap);
+}
+
 /* Active sums over the problems still running: workgroup-wide, every
  * thread gets the sums of problems before `p` (pre) and of all (tot). */
 DEV void active_sums(const hb_batch &B, int p, int pre[HB_NPH], int tot[HB_NPH], bool &p_active)
@@ -2746,14 +2785,24 @@ __global__ __launch_bounds__(HB_BLOCK) void kb_finalize(const hb_dev *__restrict
 }
 
 /* flag[0] = 1 once every problem is done; flag[1] = problems still running;
- * flag[2 + ph] = entries of phase ph's table those problems hold */
+ * flag[2 + ph] = entries of phase ph's table those problems hold; flag[2 +
+ * HB_NPH] = problems the resident form still has work for */
 __global__ __launch_bounds__(HB_BLOCK) void kb_publish(hb_batch B, int *flag)
 {
     __shared__ int cnt[HB_BLOCK];
-    int c = 0;
-    for (int q = threadIdx.x; q < B.nprob; q += HB_BLOCK) c += B.devs[q].st->done ? 0 : 1;
+    __shared__ int res;
+    int c = 0, cr = 0;
+    for (int q = threadIdx.x; q < B.nprob; q += HB_BLOCK) {
+        const hb_state *st = B.devs[q].st;
+        if (st->done) continue;
+        ++c;
+        /* one left to the launches: until the shifts have caught up */
+        if (B.devs[q].res_G && (!st->res_fail || st->k != st->ks)) ++cr;
+    }
     cnt[threadIdx.x] = c;
+    if (threadIdx.x == 0) res = 0;
     __syncthreads();
+    if (cr) atomicAdd(&res, cr);
     for (int w = HB_BLOCK / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) cnt[threadIdx.x] += cnt[threadIdx.x + w];
         __syncthreads();
@@ -2765,6 +2814,7 @@ __global__ __launch_bounds__(HB_BLOCK) void kb_publish(hb_batch B, int *flag)
         flag[0] = cnt[0] == 0;
         flag[1] = cnt[0];
         for (int ph = 0; ph < HB_NPH; ++ph) flag[2 + ph] = tot[ph];
+        flag[2 + HB_NPH] = res;
         __threadfence_system();
     }
 }
@@ -3141,6 +3191,15 @@ int hb_kb_iteration(const hb_batch *B, hipStream_t s)
         if (e) return e;
     }
     return 0;
+}
+
+int hb_kb_res_flush(const hb_batch *B, hipStream_t s)
+{
+    /* components -1 .. 2 W of every list position */
+    hipLaunchKernelGGL(kb_res_coef, dim3(B->n_coef_tiles, (2 * B->W + 2 + HB_BLOCK - 1) / HB_BLOCK), dim3(HB_BLOCK), 0,
+                       s, B->devs, B->t_coef);
+    hipLaunchKernelGGL(kb_res_flush, dim3(B->n_shift_tiles), dim3(HB_BLOCK), 0, s, B->devs, B->t_shift);
+    return (int)hipGetLastError();
 }
 
 int hb_kb_publish(const hb_batch *B, int *flag_dev, hipStream_t s)

@@ -102,6 +102,13 @@ int hb_kb_iteration(const hb_batch *B, hipStream_t s);
 int hb_kb_publish(const hb_batch *B, int *flag_dev, hipStream_t s);
 int hb_kb_compact(const hb_batch *B, hipStream_t s);
 int hb_kb_finalize(const hb_batch *B, hipStream_t s);
+/* The resident form over every problem of a batch, as the hb_k_res_ calls;
+ * shape of a problem whose workgroups take 4 SB tiles (0: does not fit). */
+int hb_k_res_shape_b(int nblk, int SB, int *lcw);
+int hb_kb_res_fill(const hb_batch *B, hipStream_t s);
+int hb_kb_res_iterations(const hb_batch *B, hipStream_t s);
+int hb_kb_res_flush(const hb_batch *B, hipStream_t s);
+int hb_kb_res_leave(const hb_batch *B, hipStream_t s);
 
 #ifdef __cplusplus
 }

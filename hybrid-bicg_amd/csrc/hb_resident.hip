@@ -119,29 +119,45 @@ DEV double shift_p(double p, double r, double s, double pb, double pbw)
  * else one per diagonal (res_val).  KT 5 and 7: exactly that many, the middle
  * one the main diagonal (the 2-D and 3-D stencils), whose x is the row's own
  * and is not gathered; 8 and 16: at most so many, in any places. */
-template <int SB, int E, int KT, bool FULL, bool SOLO>
-__global__ __launch_bounds__(RB) void k_resident(hb_dev d)
+template <int S, bool SOLO>
+struct res_lds {
+    double rh[S][RB], s[S][RB];
+    double ws[2][4 * S][4], ts[2][4 * S];
+    double x[SOLO ? S * RB : 1];   /* one workgroup: the gathered vector */
+    double ex[HB_BLOCK / 2], ep[2][HB_BLOCK / 2];
+    double red[8];
+    unsigned need[8];
+    int go;
+};
+
+/* Workgroup w of G.  WIDE: a workgroup may own more columns than it has
+ * groups of threads (lcw up to 4; batches).  D: the record by value in the
+ * kernel's arguments, or in constant memory. */
+template <int SB, int E, int KT, bool FULL, bool SOLO, bool WIDE, class D>
+DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
 {
     constexpr int DP = KT & 1 ? KT / 2 : -1;
     constexpr int S = SB * E;         /* tiles of 256 rows per group of 256 threads */
     constexpr int NT = 4 * S;         /* tiles of the workgroup */
-    __shared__ double l_rh[S][RB], l_s[S][RB];
-    __shared__ double l_ws[2][NT][4], l_ts[2][NT];
-    __shared__ double l_x[SOLO ? S * RB : 1];   /* one workgroup: the gathered vector */
-    __shared__ double l_ex[HB_BLOCK / 2], l_ep[2][HB_BLOCK / 2];
-    __shared__ double l_red[8];
-    __shared__ unsigned l_need[8];
-    __shared__ int l_go;
+    auto &l_rh = L.rh;
+    auto &l_s = L.s;
+    auto &l_ws = L.ws;
+    auto &l_ts = L.ts;
+    auto &l_x = L.x;
+    auto &l_ex = L.ex;
+    auto &l_ep = L.ep;
+    auto &l_red = L.red;
+    auto &l_need = L.need;
+    int &l_go = L.go;
 
     hb_state *st = d.st;
     const int kf = st->ks;
-    if (st->done | (st->k != kf)) return;   /* finished, or the shifts have not caught up */
+    /* finished, the shifts have not caught up, or left to the launches */
+    if (st->done | (st->k != kf) | st->res_fail) return;
     const int tid = threadIdx.x, lane = tid & 63;
     int lt = tid & 255;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2;
-    const int G = SOLO ? 1 : (int)gridDim.x;
-    const int w = SOLO ? 0 : (int)xcd_tile(blockIdx.x, gridDim.x);
     const int n = d.n, nblk = d.nblk, W = d.W, P = d.res_P;
     const int seed = st->seed, win_k0 = st->win_k0, fresh = st->res_fresh;
     int switched = st->switched;
@@ -167,17 +183,28 @@ __global__ __launch_bounds__(RB) void k_resident(hb_dev d)
      * the columns, 10 us against 5 at 128^3.
      * Slot (u, e) of group g: column w CW + g % CW, row g / CW + 4 u / CW of
      * it, and E > 1: 8 e rows further (CW = 1, SB = 2), the tiles 2048 apart
-     * that the seed update's partial sums chain.  One workgroup: tile g + 4 u. */
+     * that the seed update's partial sums chain.  CW > 4 (wh = log2(CW / 4)):
+     * the columns first, four slot by slot, then the next row.  One workgroup:
+     * tile g + 4 u. */
     const int lcw = SOLO ? 0 : d.res_lcw, CW = 1 << lcw;
+    const int wh = WIDE ? max(lcw - 2, 0) : 0, wl = lcw - wh;
     const int ncol = min(nblk, 256);
     const int tile_g = SOLO ? grp : (w << lcw) + (grp & (CW - 1)) + 256 * (grp >> lcw);
-    const int tile_u = SOLO ? 4 : 256 * (4 >> lcw);
+    const int tile_u = SOLO ? 4 : 256 * (4 >> wl);
     /* its place among the workgroup's wave sums: column by column */
     const int ws_g = SOLO ? grp : (grp & (CW - 1)) * (NT >> lcw) + (grp >> lcw);
-    const int ws_u = SOLO ? 4 : 4 >> lcw;
+    const int ws_u = SOLO ? 4 : 4 >> wl;
     int t0 = tile_g;
-    auto tile_of = [&](int sl) { return t0 + tile_u * (sl / E) + 2048 * (sl % E); };
-    auto ws_of = [&](int sl) { return ws_g + ws_u * (sl / E) + 8 * (sl % E); };
+    auto tile_of = [&](int sl) {
+        const int u = sl / E;
+        if (WIDE && !SOLO) return t0 + 4 * (u & ((1 << wh) - 1)) + tile_u * (u >> wh);
+        return t0 + tile_u * u + 2048 * (sl % E);
+    };
+    auto ws_of = [&](int sl) {
+        const int u = sl / E;
+        if (WIDE && !SOLO) return ws_g + 4 * (u & ((1 << wh) - 1)) * (NT >> lcw) + ws_u * (u >> wh);
+        return ws_g + ws_u * u + 8 * (sl % E);
+    };
     /* how many rows it has (<= 0: none), uniform across the wave; own rows
      * are base + lt, a uniform address and one constant lane offset */
     auto rows_of = [&](int sl) { return n - tile_of(sl) * HB_BLOCK; };
@@ -633,6 +660,14 @@ __global__ __launch_bounds__(RB) void k_resident(hb_dev d)
     }
 }
 
+template <int SB, int E, int KT, bool FULL, bool SOLO>
+__global__ __launch_bounds__(RB) void k_resident(hb_dev d)
+{
+    __shared__ res_lds<SB * E, SOLO> L;
+    resident_body<SB, E, KT, FULL, SOLO, false>(d, L, SOLO ? 0 : (int)xcd_tile(blockIdx.x, gridDim.x),
+                                                SOLO ? 1 : (int)gridDim.x);
+}
+
 /* ---- the shifts over the iterations a resident launch ran ---------------------
  * src/solver_dynamic.c:243-253 (per-shift recurrences), :278-303 (convergence
  * check), :312-341 (seed switch), as scalar_stage (hb_kernels.hip) does them an
@@ -646,7 +681,8 @@ struct res_shift {
     int stop_k, last_k, len, bad, spike;
 };
 
-__global__ __launch_bounds__(RB) void k_res_stage(hb_dev d)
+template <class D>
+DEV void res_stage_body(const D &d)
 {
     __shared__ double l_a[HB_RES_CMAX], l_w[HB_RES_CMAX], l_b[HB_RES_CMAX], l_ra[HB_RES_CMAX];
     __shared__ double l_nq[HB_RES_CMAX], l_nr[HB_RES_CMAX + 1], l_dr[HB_RES_CMAX];
@@ -932,18 +968,27 @@ __global__ __launch_bounds__(RB) void k_res_stage(hb_dev d)
     }
 }
 
+__global__ __launch_bounds__(RB) void k_res_stage(hb_dev d)
+{
+    res_stage_body(d);
+}
+
 /* The launch-per-phase kernels take over (a resident launch could not
  * start): the seed's p moves to where they keep it. */
-__global__ __launch_bounds__(HB_BLOCK) void k_res_leave(hb_dev d)
+template <class D>
+DEV void res_leave_body(const D &d)
 {
     hb_state *st = d.st;
     if (st->done) return;
     if (!st->res_fresh) {
         const double *p = d.pring + off(st->k % d.res_P, d.n);
         double *ps = d.p_set + off(st->seed, d.n);
-        for (int i = blockIdx.x * HB_BLOCK + threadIdx.x; i < d.n; i += gridDim.x * HB_BLOCK) ps[i] = p[i];
+        const int n = d.n;
+        for (int i = blockIdx.x * HB_BLOCK + threadIdx.x; i < n; i += gridDim.x * HB_BLOCK) ps[i] = p[i];
     }
 }
+
+__global__ __launch_bounds__(HB_BLOCK) void k_res_leave(hb_dev d) { res_leave_body(d); }
 
 /* ---- layout ------------------------------------------------------------------
  * The diagonals (column - row) of tile t (rows 256 t ...) in ascending order,
@@ -1015,23 +1060,92 @@ __global__ __launch_bounds__(HB_BLOCK) void k_res_bits(hb_dev d, unsigned short 
 
 /* The rows' values by diagonal, [tile][KT][256], read in CSR order from val
  * at every solve (a caller may change them in place). */
-__global__ __launch_bounds__(HB_BLOCK) void k_res_fill(hb_dev d)
+template <class D>
+DEV void res_fill_body(const D &d, int t)
 {
-    const int t = blockIdx.x, i = t * HB_BLOCK + threadIdx.x;
+    const int i = t * HB_BLOCK + threadIdx.x, KT = d.res_KT;
     const unsigned m = i < d.n ? d.rpres[i] : 0;
     unsigned e = i < d.n ? d.ptr[i] : 0;
-    double *out = d.rdia + (size_t)t * d.res_KT * HB_BLOCK + threadIdx.x;
-    for (int j = 0; j < d.res_KT; ++j) out[(size_t)j * HB_BLOCK] = (m >> j) & 1u ? d.val[e++] : 0.0;
+    double *out = d.rdia + (size_t)t * KT * HB_BLOCK + threadIdx.x;
+    const double *val = d.val;
+    for (int j = 0; j < KT; ++j) out[(size_t)j * HB_BLOCK] = (m >> j) & 1u ? val[e++] : 0.0;
+}
+
+__global__ __launch_bounds__(HB_BLOCK) void k_res_fill(hb_dev d) { res_fill_body(d, blockIdx.x); }
+
+/* ---- batches -----------------------------------------------------------------
+ * One launch runs every problem's iterations, each problem in a cluster of
+ * workgroups of its own that rendezvous and wait among themselves only;
+ * tab[2 b], tab[2 b + 1]: the problem of workgroup b and its place in the
+ * cluster, a cluster's workgroups side by side.  The dispatcher deals
+ * workgroups to the XCDs in order, so the clusters that do not fit the
+ * compute units at once follow as earlier ones end, and a waiting cluster is
+ * never ahead of one it keeps out.
+ *
+ * A batch took 8 launches an iteration whose workgroups each began with the
+ * dependent reads problem, record, vectors; here an iteration costs a problem
+ * its waits, about 18 us in a cluster of 16 tiles a workgroup.  48 problems
+ * of 1000 to 200000 rows: 60.9 ms a solve before, 30.4 ms so; bound by the
+ * first rounds, whose 440 workgroups take the 256 compute units twice. */
+template <int SB, int KT, bool FULL>
+DEV void resident_of(const HB_K hb_dev &d, unsigned char *lds, int w)
+{
+    if (d.res_G == 1)
+        resident_body<4, 1, KT, FULL, true, true>(d, *(res_lds<4, true> *)lds, 0, 1);
+    else
+        resident_body<SB, 1, KT, FULL, false, true>(d, *(res_lds<SB, false> *)lds, w, d.res_G);
+}
+
+template <int SB>
+__global__ __launch_bounds__(RB) void kb_resident(const hb_dev *__restrict__ devs, const int *__restrict__ tab)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char
+        lds[sizeof(res_lds<4, true>) > sizeof(res_lds<SB, false>) ? sizeof(res_lds<4, true>)
+                                                                  : sizeof(res_lds<SB, false>)];
+    const HB_K int *t = read_only(tab) + 2 * blockIdx.x;
+    const HB_K hb_dev &d = read_only(devs)[t[0]];
+    const int w = t[1];
+    switch (d.res_KT + (d.res_full ? 100 : 0)) {
+    case 5: return resident_of<SB, 5, false>(d, lds, w);
+    case 7: return resident_of<SB, 7, false>(d, lds, w);
+    case 16: return resident_of<SB, 16, false>(d, lds, w);
+    case 105: return resident_of<SB, 5, true>(d, lds, w);
+    case 107: return resident_of<SB, 7, true>(d, lds, w);
+    case 116: return resident_of<SB, 16, true>(d, lds, w);
+    }
+}
+
+__global__ __launch_bounds__(RB) void kb_res_stage(const hb_dev *__restrict__ devs)
+{
+    res_stage_body(read_only(devs)[blockIdx.x]);
+}
+
+__global__ __launch_bounds__(HB_BLOCK) void kb_res_fill(const hb_dev *__restrict__ devs, const int *__restrict__ tab)
+{
+    const HB_K int *t = read_only(tab) + 2 * blockIdx.x;
+    const HB_K hb_dev &d = read_only(devs)[t[0]];
+    if (d.res_full) res_fill_body(d, t[1]);
+}
+
+__global__ __launch_bounds__(HB_BLOCK) void kb_res_leave(const hb_dev *__restrict__ devs)
+{
+    res_leave_body(read_only(devs)[blockIdx.y]);
 }
 
 /* ---- launch layer --------------------------------------------------------- */
 template <int SB, int E, int KT, bool FULL>
 static int launch_res(const hb_dev *d, hipStream_t s)
 {
-    if (d->res_G > 1) hipLaunchKernelGGL((k_resident<SB, E, KT, FULL, false>), dim3(d->res_G), dim3(RB), 0, s, *d);
-    else if constexpr (E == 1) hipLaunchKernelGGL((k_resident<SB, E, KT, FULL, true>), dim3(1), dim3(RB), 0, s, *d);
-    else return -1;
-    return (int)hipGetLastError();
+    if (d->res_G > 1) {
+        if constexpr (SB < 4) {
+            hipLaunchKernelGGL((k_resident<SB, E, KT, FULL, false>), dim3(d->res_G), dim3(RB), 0, s, *d);
+            return (int)hipGetLastError();
+        }
+    } else if constexpr (E == 1) {
+        hipLaunchKernelGGL((k_resident<SB, E, KT, FULL, true>), dim3(1), dim3(RB), 0, s, *d);
+        return (int)hipGetLastError();
+    }
+    return -1;
 }
 
 template <int SB, int E>
@@ -1070,6 +1184,40 @@ int hb_k_res_shape(int nblk, int cus, int *SB, int *E, int *lcw)
     if (nblk > 2048) *E = nblk <= 4096 ? 2 : 4;
     const int G = ((nblk < 256 ? nblk : 256) + (1 << *lcw) - 1) >> *lcw;
     return nblk <= 8192 && G <= cus ? G : 0;
+}
+
+/* A problem of a batch whose workgroups take 4 SB tiles: its workgroups (one
+ * up to 16 tiles), 0 where the rows do not fit; lcw up to 4. */
+int hb_k_res_shape_b(int nblk, int SB, int *lcw)
+{
+    *lcw = 0;
+    if (nblk <= 16) return 1;
+    const int rows = (nblk + 255) / 256;   /* tiles of a column */
+    if (rows > 4 * SB || nblk > 2048) return 0;
+    while ((rows << (*lcw + 1)) <= 4 * SB) ++*lcw;
+    return ((nblk < 256 ? nblk : 256) + (1 << *lcw) - 1) >> *lcw;
+}
+
+int hb_kb_res_iterations(const hb_batch *B, hipStream_t s)
+{
+    const dim3 g(B->n_res), bl(RB);
+    if (B->res_SB == 1) hipLaunchKernelGGL(kb_resident<1>, g, bl, 0, s, B->devs, B->t_res);
+    else if (B->res_SB == 2) hipLaunchKernelGGL(kb_resident<2>, g, bl, 0, s, B->devs, B->t_res);
+    else hipLaunchKernelGGL(kb_resident<4>, g, bl, 0, s, B->devs, B->t_res);
+    hipLaunchKernelGGL(kb_res_stage, dim3(B->nprob), bl, 0, s, B->devs);
+    return (int)hipGetLastError();
+}
+
+int hb_kb_res_fill(const hb_batch *B, hipStream_t s)
+{
+    hipLaunchKernelGGL(kb_res_fill, dim3(B->n_spmv_tiles), dim3(HB_BLOCK), 0, s, B->devs, B->t_spmv);
+    return (int)hipGetLastError();
+}
+
+int hb_kb_res_leave(const hb_batch *B, hipStream_t s)
+{
+    hipLaunchKernelGGL(kb_res_leave, dim3(64, B->nprob), dim3(HB_BLOCK), 0, s, B->devs);
+    return (int)hipGetLastError();
 }
 
 int hb_k_res_scan(const hb_dev *d, int *tK, int *toff, int *bad, hipStream_t s)

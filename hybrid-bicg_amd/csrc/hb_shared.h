@@ -257,6 +257,8 @@ typedef struct hb_batch {
     int *act;                  /* [HB_NPH] entries in each active list     */
     const int *pofs;           /* [HB_NPH][nprob] problem p's first entry in each full table */
     const int *pcnt;           /* [HB_NPH][nprob] and its entries          */
+    const int *t_res;          /* [2*n_res] (problem, workgroup of its cluster): resident form */
+    int n_res, res_SB;         /* its workgroups; tiles per group of 256 threads */
     int div;                   /* the phase launches take ceil(full / div) workgroups */
 } hb_batch;
 

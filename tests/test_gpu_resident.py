@@ -8,7 +8,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
-from hbicg import Plan, make_params
+from hbicg import Batch, Plan, make_params
 from hbicg import problems as P
 
 pytestmark = pytest.mark.gpu
@@ -132,6 +132,52 @@ def test_hand_over(M, seed):
     kernel and in a launch of its own)"""
     A = P.conv_diff_2d(90, 81, 4.01)
     _same(_run(A, M, seed, fused=4), _run(A, M, seed, fused=0))
+
+
+def _batch(mats, **kw):
+    """Two solves of a batch of matrices, problem i with 1 + 5 i mod 37 shifts."""
+    dev = "cuda"
+    spec = []
+    for i, A in enumerate(mats):
+        M = 1 + 5 * i % 37
+        spec.append({"val": torch.as_tensor(A.val).to(dev), "col": torch.as_tensor(A.col.view(np.int32)).to(dev),
+                     "ptr": torch.as_tensor(A.ptr.view(np.int32)).to(dev),
+                     "b": torch.as_tensor(P.uniform(i, 1, A.n, -1.0, 1.0)).to(dev),
+                     "sigma": P.logspace_shifts(M, 1e-3, 1.0), "seed": M // 2 if i % 3 else 0})
+    bt = Batch(None, make_params(tol=1e-10, graph=1, **kw), device_spec=spec)
+    out = []
+    for _ in range(2):
+        k, xs, _ = bt.solve()
+        for i in range(len(mats)):
+            rep, stop, sw = bt.report(i)
+            out.append((int(k[i]), xs[i].clone(), torch.zeros(1), stop.copy(), list(sw), rep["status"], None))
+    bt.close()
+    return out
+
+
+_T = 256
+
+
+@pytest.mark.parametrize("kw", [{}, dict(window=17, growth_limit=30.0), dict(fused=4), dict(window=9)])
+@pytest.mark.parametrize("sizes", [
+    [1, 63, 256, 257, 1000, 4 * _T, 4 * _T + 3, 16 * _T, 16 * _T + 1],        # one workgroup, and the first of two
+    [17 * _T - 1, 63 * _T + 77, 64 * _T, 255 * _T, 256 * _T + 9, 20 * _T],    # one tile a column, and one more
+    [513 * _T - 100, 300 * _T, 900 * _T + 1, 1024 * _T, 600 * _T],            # up to four
+    [1025 * _T, 2048 * _T - 1, 100 * _T, 2],                                  # up to eight
+    [2049 * _T, 100 * _T, 2],                                                 # one that does not fit
+])
+def test_batch(sizes, kw):
+    """clusters of one to many workgroups (all sizes of their columns), next
+    to each other; more of them than compute units"""
+    mats = [_banded(n, ([0], [-1, 0, 1], [-7, -1, 0, 1, 7], [-40, -6, -1, 0, 1, 6, 40],
+                        [-5, 1, 0, 7, 8, 9, 11, 300])[i % 5] if n > 300 else [-1, 0, 1], i,
+                    "full" if i % 2 else "const") for i, n in enumerate(sizes)]
+    _same(_batch(mats, **kw), _batch(mats, **{**kw, "fused": 0}))
+
+
+def test_batch_more_clusters_than_compute_units():
+    mats = [P.conv_diff_2d(60 + i % 50, 70, 4.01) for i in range(320)]
+    _same(_batch(mats), _batch(mats, fused=0))
 
 
 def test_values_in_place():
