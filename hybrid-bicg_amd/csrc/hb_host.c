@@ -130,6 +130,9 @@ struct hbicg_plan {
     int *stop, *stop_iter, *act_len, *flist, *fpos, *switch_k, *switch_to;
     hb_state *st;
     int *flag_host;      /* pinned: {done, k, res_fail, ks} */
+    double *sig_host;    /* pinned, with it: the call's shifts [M], residuals [M], */
+    double *res_host;
+    int *out_host;       /* what the last launch reports (hb_dev.out)              */
     hipEvent_t ev[2], t0, t1;
     /* resident form: layout, ring of p, logs, mailboxes (hb_resident.hip) */
     int *rend;
@@ -877,7 +880,11 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
     if (rc) goto fail;
     /* unused combined-coefficient columns stay finite */
     HIPCK(hipMemset(pl->ccoef, 0, ccn * 8));
-    HIPCK(hipHostMalloc((void **)&pl->flag_host, 4 * sizeof(int), hipHostMallocDefault));
+    HIPCK(hipHostMalloc((void **)&pl->flag_host, 4 * sizeof(int) + (size_t)M * 28 + sizeof(hb_state),
+                        hipHostMallocDefault));
+    pl->sig_host = (double *)(pl->flag_host + 4);
+    pl->res_host = pl->sig_host + M;
+    pl->out_host = (int *)(pl->res_host + M);
     HIPCK(hipEventCreateWithFlags(&pl->ev[0], hipEventDisableTiming));
     HIPCK(hipEventCreateWithFlags(&pl->ev[1], hipEventDisableTiming));
     HIPCK(hipEventCreate(&pl->t0));
@@ -894,6 +901,8 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
     d->vec_grid = vec_grid;
     d->shift_gx = gx; d->shift_gy = gy; d->shift_group = G; d->vec2 = vec2;
     d->x_zero = p->x_zero != 0;
+    d->sig_in = pl->sig_host;
+    d->out = pl->out_host;
     pl->vec2 = vec2;
     d->tol = pl->tol;
     d->growth_limit = pl->growth_limit;
@@ -1159,6 +1168,16 @@ fail:
     return rc;
 }
 
+/* what the finished solve left in pinned memory */
+static void read_out(hbicg_plan *pl, hb_state *st)
+{
+    const size_t words = sizeof(*st) / 4, M = (size_t)pl->M;
+    memcpy(st, pl->out_host, sizeof(*st));
+    memcpy(pl->h_stop_iter, pl->out_host + words, M * 4);
+    memcpy(pl->h_switch_k, pl->out_host + words + M, M * 4);
+    memcpy(pl->h_switch_to, pl->out_host + words + 2 * M, M * 4);
+}
+
 static int run_loop(hbicg_plan *pl)
 {
     int rc = 0;
@@ -1224,8 +1243,7 @@ int hbicg_plan_solve(hbicg_plan *pl, const double *b, const double *sigma, int s
     pl->dev.x_set = dx;
     /* 16-byte accesses in the shift kernel need an aligned x_set */
     pl->dev.vec2 = pl->vec2 && ((((size_t)dx) & 15) == 0);
-    HIPCK(hipMemcpyAsync(pl->sigma, sigma, (size_t)pl->M * 8, hipMemcpyHostToDevice, pl->stream));
-    HIPCK(hipMemsetAsync(pl->st, 0, sizeof(hb_state), pl->stream));
+    memcpy(pl->sig_host, sigma, (size_t)pl->M * 8);
     HIPCK(hipEventRecord(pl->t0, pl->stream));
     pl->dev.b_in = db;
     pl->dev.seed_in = seed;
@@ -1246,18 +1264,15 @@ int hbicg_plan_solve(hbicg_plan *pl, const double *b, const double *sigma, int s
     HIPCK(hipEventRecord(pl->t1, pl->stream));
 
     hb_state st;
-    HIPCK(hipMemcpyAsync(&st, pl->st, sizeof(st), hipMemcpyDeviceToHost, pl->stream));
     HIPCK(hipStreamSynchronize(pl->stream));
+    read_out(pl, &st);
     const double *r_dev = pl->rring + (size_t)(st.kprev % (pl->W + 1)) * pl->n;
     if (r_out) {
         if (on_device) HIPCK(hipMemcpyAsync(r_out, r_dev, nb, hipMemcpyDeviceToDevice, pl->stream));
         else HIPCK(hipMemcpyAsync(r_out, r_dev, nb, hipMemcpyDeviceToHost, pl->stream));
     }
     if (!on_device) HIPCK(hipMemcpyAsync(x_set, dx, xb, hipMemcpyDeviceToHost, pl->stream));
-    HIPCK(hipMemcpyAsync(pl->h_stop_iter, pl->stop_iter, (size_t)pl->M * 4, hipMemcpyDeviceToHost, pl->stream));
-    HIPCK(hipMemcpyAsync(pl->h_switch_k, pl->switch_k, (size_t)pl->M * 4, hipMemcpyDeviceToHost, pl->stream));
-    HIPCK(hipMemcpyAsync(pl->h_switch_to, pl->switch_to, (size_t)pl->M * 4, hipMemcpyDeviceToHost, pl->stream));
-    HIPCK(hipStreamSynchronize(pl->stream));
+    if (r_out || !on_device) HIPCK(hipStreamSynchronize(pl->stream));
     float ms = 0.0f;
     HIPCK(hipEventElapsedTime(&ms, pl->t0, pl->t1));
 
@@ -1399,7 +1414,7 @@ int hbicg_plan_true_residuals(hbicg_plan *pl, const double *b, const double *sig
                               const double *x_set, int on_device, double *out)
 {
     int rc = 0;
-    double *part = NULL, *dout = NULL;
+    double *part = NULL;
     if (!pl || !b || !sigma || !x_set || !out) return HBICG_E_ARG;
     HIPCK(hipSetDevice(pl->device));
     const size_t nb = (size_t)pl->n * 8, xb = nb * (size_t)pl->M;
@@ -1417,18 +1432,16 @@ int hbicg_plan_true_residuals(hbicg_plan *pl, const double *b, const double *sig
     HIPCK(hipMemcpyAsync(pl->sigma, sigma, (size_t)pl->M * 8, hipMemcpyHostToDevice, pl->stream));
     const int R = hb_k_resid_blocks(pl->n, pl->M);
     part = (double *)dalloc((size_t)R * pl->M * 2 * 8, &rc);
-    dout = (double *)dalloc((size_t)pl->M * 8, &rc);
     if (rc) goto fail;
-    if (hb_k_true_residual(&pl->dev, db, pl->sigma, dx, part, dout, pl->stream) != 0) {
+    if (hb_k_true_residual(&pl->dev, db, pl->sigma, dx, part, pl->res_host, pl->stream) != 0) {
         rc = HBICG_E_HIP;
         goto fail;
     }
-    HIPCK(hipMemcpyAsync(out, dout, (size_t)pl->M * 8, hipMemcpyDeviceToHost, pl->stream));
     HIPCK(hipStreamSynchronize(pl->stream));
+    memcpy(out, pl->res_host, (size_t)pl->M * 8);
 fail:
     if (rc) hipStreamSynchronize(pl->stream);
     hb_pool_put(part);
-    hb_pool_put(dout);
     return rc;
 }
 
@@ -1966,8 +1979,7 @@ static int batch_run(hbicg_batch *bt, const double *const *b, const double *cons
         d->cap = max_iter_override > 0 ? max_iter_override + 1 : pl->cap;
         if (d->cap > pl->cap) d->cap = pl->cap;
         if (d->cap > max_cap) max_cap = d->cap;
-        HIPCK(hipMemcpyAsync(pl->sigma, sigma[p], (size_t)pl->M * 8, hipMemcpyHostToDevice, bt->stream));
-        HIPCK(hipMemsetAsync(pl->st, 0, sizeof(hb_state), bt->stream));
+        memcpy(pl->sig_host, sigma[p], (size_t)pl->M * 8);
     }
     HIPCK(hipMemcpyAsync(bt->ddevs, bt->hdevs, (size_t)bt->nprob * sizeof(hb_dev), hipMemcpyHostToDevice,
                          bt->stream));
@@ -2020,11 +2032,7 @@ int hbicg_batch_solve(hbicg_batch *bt, const double *const *b, const double *con
     for (int p = 0; p < bt->nprob; ++p) {
         hbicg_plan *pl = bt->plans[p];
         hb_state st;
-        HIPCK(hipMemcpyAsync(&st, pl->st, sizeof(st), hipMemcpyDeviceToHost, bt->stream));
-        HIPCK(hipMemcpyAsync(pl->h_stop_iter, pl->stop_iter, (size_t)pl->M * 4, hipMemcpyDeviceToHost, bt->stream));
-        HIPCK(hipMemcpyAsync(pl->h_switch_k, pl->switch_k, (size_t)pl->M * 4, hipMemcpyDeviceToHost, bt->stream));
-        HIPCK(hipMemcpyAsync(pl->h_switch_to, pl->switch_to, (size_t)pl->M * 4, hipMemcpyDeviceToHost, bt->stream));
-        HIPCK(hipStreamSynchronize(bt->stream));
+        read_out(pl, &st);
         hbicg_report *R = &pl->rep;
         memset(R, 0, sizeof(*R));
         R->k = st.k;
@@ -2048,8 +2056,6 @@ int hbicg_batch_solve(hbicg_batch *bt, const double *const *b, const double *con
     }
     if (solve_ms) *solve_ms = bt->last_ms;
     return 0;
-fail:
-    return rc;
 }
 
 int hbicg_batch_report(hbicg_batch *bt, int p, hbicg_report *rep, int *stop_iter,

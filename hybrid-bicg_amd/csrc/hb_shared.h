@@ -233,6 +233,10 @@ typedef struct hb_dev {
     HB_G const double *b_in;   /* right-hand side read by the initialisation */
     int seed_in;               /* first seed                               */
     int pad_;
+    /* pinned host memory, so that a solve needs no small copies: */
+    HB_G const double *sig_in; /* [M] the call's shifts; the initialisation moves them to sigma */
+    HB_G int *out;             /* where the last launch leaves the state, then stop_iter,
+                                  switch_k and switch_to [M each]          */
 } hb_dev;
 
 /* A batch of independent problems: per-problem hb_dev records in device
