@@ -671,15 +671,28 @@ __global__ __launch_bounds__(RB) void k_resident(hb_dev d)
 /* ---- the shifts over the iterations a resident launch ran ---------------------
  * src/solver_dynamic.c:243-253 (per-shift recurrences), :278-303 (convergence
  * check), :312-341 (seed switch), as scalar_stage (hb_kernels.hip) does them an
- * iteration at a time.  Between switches no shift depends on another, so a
- * thread takes its shift through all the iterations without a barrier.  The
- * growth guard can close the window inside the range: the threads then run
- * again up to that iteration (the recurrences do not depend on the window),
- * and the next launch takes the rest. */
+ * iteration at a time.  Between switches no shift depends on another; what
+ * an iteration hands to the next is pi, eta and zeta (three dependent
+ * operations) and the growth bound (two), while the coefficients, with
+ * their six divisions, are most of the work.  So of T = 1024 / M iterations
+ * at a time a shift's owner thread runs the recurrences, every thread then
+ * forms one (shift, iteration)'s coefficients, and the owner goes through
+ * them for the bound and the stopping rule.  A thread taking its shift
+ * through everything, and the switch's replay from memory, took 445 us of a
+ * 251 x 173 solve (23 shifts, 394 iterations) and 107 of a 64 x 64 one (16,
+ * 108); so 284 and 63.
+ * The growth guard can close the window inside the range: all of it then
+ * runs again up to that iteration (the recurrences do not depend on the
+ * window), and the next launch takes the rest. */
 struct res_shift {
     double eta, zeta, grow, own, zp;
     int stop_k, last_k, len, bad, spike;
 };
+
+/* bits of one (shift, iteration) */
+#define RES_F_BAD   1   /* a divisor is 0 or not finite   */
+#define RES_F_STOP  2   /* the shift has converged         */
+#define RES_F_ABOVE 4   /* its estimate is above the seed's */
 
 template <class D>
 DEV void res_stage_body(const D &d)
@@ -689,6 +702,10 @@ DEV void res_stage_body(const D &d)
     __shared__ double sh_zp[RB];
     __shared__ int sh_j[RB], sh_k[RB], sh_n[RB];
     __shared__ int sh_spike, sh_bad;
+    /* T iterations of up to 1024 shifts: pi and the zeta before, the bound's
+     * terms, the pi ahead of the first; sh_zp, sh_n: estimates and bits;
+     * sh_j, sh_k: a shift's place in the flush list (-1: it has stopped) */
+    __shared__ double sh_pi[RB], sh_z[RB], sh_b[RB], sh_o[RB], sh_p0[RB], sh_dj[RB];
     hb_state *st = d.st;
     const int tid = threadIdx.x, M = d.M;
     if (tid == 0) {
@@ -714,7 +731,7 @@ DEV void res_stage_body(const D &d)
         l_a[i] = d.aa[k];
         l_w[i] = d.wa[k];
         l_b[i] = d.ba[k];
-        l_ra[i] = d.ba[k - 1] / d.aa[k - 1];
+        l_ra[i] = d.ba[k - 1] / d.aa[k - 1] * d.aa[k];
         l_nq[i] = sqrt(d.qqlog[k]);
         l_nr[i + 1] = sqrt(dr);
         l_dr[i] = dr;
@@ -750,70 +767,104 @@ DEV void res_stage_body(const D &d)
     }
     __syncthreads();
 
-    auto walk = [&](int j, int kend) -> res_shift {
-        res_shift z;
-        z.eta = d.eta[j];
-        z.zeta = d.zeta[j];
-        z.grow = d.growth_limit > 0.0 ? d.grow[j] : 0.0;
-        z.own = d.growth_limit > 0.0 ? d.grow[M + j] : 0.0;
+    /* shifts c0 .. of at most 1024, each its thread's in z, up to kend */
+    auto walk = [&](int c0, int kend, res_shift &z) {
+        const int Mc = min(M - c0, RB), T = RB / Mc, bt = tid / Mc, bj = tid - bt * Mc;
+        const int j = c0 + tid;
+        bool live = tid < Mc && j != s && !d.stop[j];
+        double pim1 = 1.0;
         z.zp = 0.0;
         z.stop_k = 0; z.last_k = 0; z.len = 0; z.bad = 0; z.spike = INT_MAX;
-        const double dj = sig_s - d.sigma[j];
-        const int pos = d.fpos[j];
-        double pim1 = PI(d, j, k0 - 1);
-        for (int k = k0; k <= kend; ++k) {
-            const int i = k - k0;
-            const double ak = l_a[i], wk = l_w[i], beta = l_b[i];
-            const double eta = l_ra[i] * ak * z.eta - dj * ak * pim1;
-            const double pik = eta + pim1;
-            const double aj = (pim1 / pik) * ak;
-            const double den = 1.0 - wk * dj;
-            if (!(den != 0.0 && isfinite(den) && pik != 0.0 && isfinite(pik))) z.bad = 1;
-            const double wj = wk / den;
-            const double zj = z.zeta;
-            const double az = aj * zj;
-            const double c1 = wj / (pik * zj);
-            const double c2 = wj / (az * pik);
-            const double c3 = -wj / (az * pim1);
-            const double znew = den * zj;
-            const double t = pim1 / pik;
-            const double bj = t * t * beta;
-            const double c4 = 1.0 / (pik * znew);
-            PI(d, j, k) = pik;
-            double *c = d.coef + ((size_t)(k - win_k0) * M + pos) * 6;
-            c[0] = c1; c[1] = aj; c[2] = c2; c[3] = c3; c[4] = bj; c[5] = c4;
-            if (d.growth_limit > 0.0) {
-                const double nrn = l_nr[i + 1];
-                const double own = fabs(bj) * (fabs(c2) * l_nq[i] + fabs(c3) * l_nr[i]) + fabs(c4) * nrn;
-                const double prev = k == 1 ? sqrt(dot_zero) : z.grow;
-                const double bound = fabs(bj) * prev + own;
-                if (!(bound <= d.growth_limit * own) && z.spike == INT_MAX) z.spike = k;
-                z.grow = bound;
-                z.own = own;
-            }
-            z.eta = eta;
-            z.zeta = znew;
-            z.len = k - win_k0 + 1;
-            const double zp = fabs(1.0 / (znew * pik));
-            if (d.trace) d.trace[(size_t)k * M + j] = zp * sqrt(l_dr[i] / dot_zero);
-            if (zp * zp * l_dr[i] <= thr) {
-                z.stop_k = k;
-                break;
-            } else if (zp > 1.0) {
-                z.last_k = k;
-                z.zp = zp;
-            }
-            pim1 = pik;
+        if (tid < Mc) {
+            sh_j[tid] = live ? d.fpos[j] : -1;
+            sh_dj[tid] = sig_s - d.sigma[j];
         }
-        return z;
+        if (live) {
+            z.eta = d.eta[j];
+            z.zeta = d.zeta[j];
+            z.grow = d.growth_limit > 0.0 ? d.grow[j] : 0.0;
+            z.own = d.growth_limit > 0.0 ? d.grow[M + j] : 0.0;
+            pim1 = PI(d, j, k0 - 1);
+        }
+        for (int kc = k0; kc <= kend; kc += T) {
+            const int nt = min(T, kend - kc + 1);
+            if (live) {
+                const double dj = sh_dj[tid];
+                sh_p0[tid] = pim1;
+#pragma unroll 4
+                for (int t = 0; t < nt; ++t) {
+                    const int i = kc - k0 + t;
+                    z.eta = l_ra[i] * z.eta - dj * l_a[i] * pim1;
+                    pim1 = z.eta + pim1;
+                    sh_pi[t * Mc + tid] = pim1;
+                    sh_z[t * Mc + tid] = z.zeta;
+                    z.zeta = (1.0 - l_w[i] * dj) * z.zeta;
+                    PI(d, j, kc + t) = pim1;
+                }
+            }
+            __syncthreads();
+            if (bt < nt && sh_j[bj] >= 0) {
+                const int k = kc + bt, i = k - k0;
+                const double dj = sh_dj[bj], ak = l_a[i], wk = l_w[i], beta = l_b[i];
+                const double pik = sh_pi[tid], pm1 = bt ? sh_pi[tid - Mc] : sh_p0[bj];
+                const double aj = (pm1 / pik) * ak;
+                const double den = 1.0 - wk * dj;
+                int f = !(den != 0.0 && isfinite(den) && pik != 0.0 && isfinite(pik)) ? RES_F_BAD : 0;
+                const double wj = wk / den;
+                const double zj = sh_z[tid];
+                const double az = aj * zj;
+                const double c1 = wj / (pik * zj);
+                const double c2 = wj / (az * pik);
+                const double c3 = -wj / (az * pm1);
+                const double znew = den * zj;
+                const double t = pm1 / pik;
+                const double bb = t * t * beta;
+                const double c4 = 1.0 / (pik * znew);
+                double *c = d.coef + ((size_t)(k - win_k0) * M + sh_j[bj]) * 6;
+                c[0] = c1; c[1] = aj; c[2] = c2; c[3] = c3; c[4] = bb; c[5] = c4;
+                sh_b[tid] = fabs(bb);
+                sh_o[tid] = fabs(bb) * (fabs(c2) * l_nq[i] + fabs(c3) * l_nr[i]) + fabs(c4) * l_nr[i + 1];
+                const double zp = fabs(1.0 / (znew * pik));
+                sh_zp[tid] = zp;
+                if (zp * zp * l_dr[i] <= thr) f |= RES_F_STOP;
+                else if (zp > 1.0) f |= RES_F_ABOVE;
+                sh_n[tid] = f;
+            }
+            __syncthreads();
+            if (live) {
+                for (int t = 0; t < nt; ++t) {
+                    const int k = kc + t, e = t * Mc + tid, f = sh_n[e];
+                    if (f & RES_F_BAD) z.bad = 1;
+                    if (d.growth_limit > 0.0) {
+                        const double own = sh_o[e];
+                        const double prev = k == 1 ? sqrt(dot_zero) : z.grow;
+                        const double bound = sh_b[e] * prev + own;
+                        if (!(bound <= d.growth_limit * own) && z.spike == INT_MAX) z.spike = k;
+                        z.grow = bound;
+                        z.own = own;
+                    }
+                    z.len = k - win_k0 + 1;
+                    if (d.trace) d.trace[(size_t)k * M + j] = sh_zp[e] * sqrt(l_dr[k - k0] / dot_zero);
+                    if (f & RES_F_STOP) {
+                        z.stop_k = k;
+                        live = false;
+                        sh_j[tid] = -1;
+                        break;
+                    } else if (f & RES_F_ABOVE) {
+                        z.last_k = k;
+                        z.zp = sh_zp[e];
+                    }
+                }
+            }
+        }
+        __syncthreads();
     };
 
     int kend = ks - 1;
     res_shift z;
     for (int pass = 0; pass < 2; ++pass) {
-        for (int j = tid; j < M; j += RB) {
-            if (j == s || d.stop[j]) continue;
-            z = walk(j, kend);
+        for (int c0 = 0; c0 < M; c0 += RB) {
+            walk(c0, kend, z);
             if (z.spike <= kend) atomicMin(&sh_spike, z.spike);
         }
         __syncthreads();
@@ -828,7 +879,10 @@ DEV void res_stage_body(const D &d)
     /* what the iterations up to kend did to the shifts */
     int nconv = 0, bk = 0, bj = -1;
     double bz = 1.0;
-    for (int j = tid; j < M; j += RB) {
+    for (int c0 = 0; c0 < M; c0 += RB) {
+        const int j = c0 + tid;
+        if (M > RB) walk(c0, kend, z);
+        if (j >= M) continue;
         if (j == s) {
             /* the seed in its own list: the recurrence at sigma_j = sigma_s */
             if (stop_s) continue;
@@ -848,7 +902,6 @@ DEV void res_stage_body(const D &d)
             continue;
         }
         if (d.stop[j]) continue;
-        if (M > RB) z = walk(j, kend);
         if (z.stop_k) {
             d.stop[j] = 1;
             d.stop_iter[j] = z.stop_k;
@@ -910,19 +963,36 @@ DEV void res_stage_body(const D &d)
         }
         __syncthreads();
         const double sig_m = d.sigma[m];
-        for (int j = tid; j < M; j += RB) {
-            double e = 0.0, z1 = 1.0;
-            if (!d.stop[j] && j != m) {
-                const double dm = sig_m - d.sigma[j];
-                for (int i = 1; i <= k; ++i) {
-                    const double pm1 = PI(d, j, i - 1);
-                    e = (d.ba[i - 1] / d.aa[i - 1]) * d.aa[i] * e - dm * d.aa[i] * pm1;
-                    PI(d, j, i) = e + pm1;
-                    z1 = (1.0 - d.wa[i] * dm) * z1;
+        for (int c0 = 0; c0 < M; c0 += RB) {
+            const int j = c0 + tid;
+            const bool run = j < M && !d.stop[j] && j != m;
+            const double dm = j < M ? sig_m - d.sigma[j] : 0.0;
+            double e = 0.0, z1 = 1.0, pim1 = run ? PI(d, j, 0) : 1.0;
+            /* the archives through LDS: read where they lie, an iteration
+             * was two dependent trips to memory and a division, 0.6 us */
+            for (int i0 = 1; i0 <= k; i0 += HB_RES_CMAX) {
+                const int ni = min(HB_RES_CMAX, k + 1 - i0);
+                __syncthreads();
+                for (int i = tid; i < ni; i += RB) {
+                    const double a = d.aa[i0 + i];
+                    l_a[i] = a;
+                    l_w[i] = d.wa[i0 + i];
+                    l_ra[i] = d.ba[i0 + i - 1] / d.aa[i0 + i - 1] * a;
+                }
+                __syncthreads();
+                if (!run) continue;
+#pragma unroll 4
+                for (int i = 0; i < ni; ++i) {
+                    e = l_ra[i] * e - dm * l_a[i] * pim1;
+                    pim1 = e + pim1;
+                    PI(d, j, i0 + i) = pim1;
+                    z1 = (1.0 - l_w[i] * dm) * z1;
                 }
             }
-            d.eta[j] = e;
-            d.zeta[j] = z1;
+            if (j < M) {
+                d.eta[j] = e;
+                d.zeta[j] = z1;
+            }
         }
     }
     /* a wait that ran out voids the solve: it ends here */
