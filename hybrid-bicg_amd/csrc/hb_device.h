@@ -149,4 +149,59 @@ DEV unsigned xcd_tile(unsigned b, unsigned nb)
 }
 
 
+/* ---- sums over a wavefront without LDS ---------------------------------------
+ * wave_sum adds, for o = 32, 16, 8, 4, 2, 1, lane i ^ o to lane i.  Addition
+ * commutes, so any exchange that pairs the same lanes gives the same bits:
+ * the gfx950 half and row swaps for 32 and 16 (which also let two values
+ * share a step), DPP for the rest.  A wave_sum through __shfl_xor is twelve
+ * LDS permutes; eight tiles' sums of a 1024-thread workgroup took longer
+ * than the SpMV that fed them. */
+template <int CTRL>
+DEV double dpp(double v)
+{
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true);
+    hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+/* sum over each row of 16 lanes: o = 8, 4, 2, 1 */
+DEV double row_sum(double v)
+{
+    v += dpp<0x128>(v);                /* row_ror:8  = i ^ 8 */
+    v += dpp<0x1b>(dpp<0x141>(v));     /* half mirror (i ^ 7), quad 3,2,1,0 (i ^ 3): i ^ 4 */
+    v += dpp<0x4e>(v);                 /* quad 2,3,0,1: i ^ 2 */
+    v += dpp<0xb1>(v);                 /* quad 1,0,3,2: i ^ 1 */
+    return v;
+}
+
+/* lanes below 32: a's halves added; the others: b's */
+DEV double swap32_add(double a, double b)
+{
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+
+/* even rows of 16 lanes: a's row pairs added; odd rows: b's */
+DEV double swap16_add(double a, double b)
+{
+    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+
+/* wave sums of two values: every lane below 32 gets a's, the others b's */
+DEV double wave_sum2(double a, double b)
+{
+    const double v = swap32_add(a, b);
+    return row_sum(swap16_add(v, v));
+}
+
+/* wave sums of four values: rows 0..3 of 16 lanes get a's, c's, b's, d's */
+DEV double wave_sum4(double a, double b, double c, double d)
+{
+    return row_sum(swap16_add(swap32_add(a, b), swap32_add(c, d)));
+}
+
 #endif

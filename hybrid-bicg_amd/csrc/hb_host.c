@@ -717,6 +717,7 @@ static int setup_resident(hbicg_plan *pl, const unsigned *hblk, int join, int ba
     for (int j = 0; j < K; ++j) {
         if (pat[j] != pat[HB_DIAG_K + j]) full = 1;
         memcpy(&d->res_val[j], &pat[j], 8);
+        if (!isfinite(d->res_val[j])) full = 1;   /* a missing entry's product has to be 0 */
     }
     for (int j = full ? 0 : K; j < HB_DIAG_K; ++j) d->res_val[j] = 0.0;
     int C = (int)(((size_t)256 << 20) / ((size_t)n * 8));

@@ -40,6 +40,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <type_traits>
 #include "hb_shared.h"
 #include "hb_launch.h"
 #include "hb_device.h"
@@ -2536,7 +2537,15 @@ __global__ void k_publish(const hb_state *st, int *flag)
  * squared entries go to one partial pair per workgroup and shift, combined in
  * a fixed order per shift.  R depends only on (n, M), so every caller gets
  * the same roundings.  An entry of A is read once for the group, not once
- * per shift, and the groups of the same rows run side by side. */
+ * per shift, and the groups of the same rows run side by side.
+ *
+ * 256 rows' entries go through LDS, as long as there are at most HB_NNZ_CAP:
+ * read by the threads that own the rows, whose entries lie 56 bytes and more
+ * apart, a load of the values touched 28 lines, and the sums of rows of
+ * several lengths selected in every step; the eight shifts' partial sums take
+ * one barrier.  96^3 rows x 48 shifts: 307 -> 260 us (340 MB of x, 68 us at
+ * a copy's rate; groups of the same rows on one XCD, or a group's rows on
+ * one, measured no faster: 413 and 373 against 345 us a call). */
 #define HB_RJ 8
 
 __global__ __launch_bounds__(HB_BLOCK) void k_resid_part(hb_dev d, const double *__restrict__ b,
@@ -2555,51 +2564,85 @@ __global__ __launch_bounds__(HB_BLOCK) void k_resid_part(hb_dev d, const double 
     double e2[HB_RJ], b2 = 0.0;
 #pragma unroll
     for (int u = 0; u < HB_RJ; ++u) e2[u] = 0.0;
-    for (int i = wg * HB_BLOCK + threadIdx.x; i < n; i += R * HB_BLOCK) {
+    __shared__ double l_val[HB_NNZ_CAP];
+    __shared__ unsigned l_col[HB_NNZ_CAP];
+    for (int r0 = wg * HB_BLOCK; r0 < n; r0 += R * HB_BLOCK) {
+        const int i = r0 + (int)threadIdx.x;
+        const unsigned t0 = ptr[r0], N = ptr[min(r0 + HB_BLOCK, n)] - t0;
+        const bool staged = N <= HB_NNZ_CAP;
+        if (staged) {
+            __syncthreads();
+            for (unsigned e = threadIdx.x; e < N; e += HB_BLOCK) {
+                l_val[e] = val[t0 + e];
+                l_col[e] = col[t0 + e];
+            }
+            __syncthreads();
+        }
+        if (i >= n) continue;
         double t[HB_RJ];
 #pragma unroll
         for (int u = 0; u < HB_RJ; ++u) t[u] = 0.0;
+        unsigned e = ptr[i];
         const unsigned e1 = ptr[i + 1];
-        for (unsigned e = ptr[i]; e < e1; e += 4) {
-            /* four entries' values, columns and gathers in flight */
-            double a[4];
-            unsigned c[4];
+        /* Q entries' gathers for all shifts in flight */
+        auto add = [&](auto Q, const double *av, const unsigned *cv, unsigned f) {
+            constexpr int q1 = decltype(Q)::value;
+            double a[q1], xv[HB_RJ][q1];
+            unsigned c[q1];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const unsigned f = min(e + q, e1 - 1);
-                a[q] = val[f];
-                c[q] = col[f];
+            for (int q = 0; q < q1; ++q) {
+                a[q] = av[f + q];
+                c[q] = cv[f + q];
             }
 #pragma unroll
             for (int u = 0; u < HB_RJ; ++u) {
                 const double *__restrict__ x = x_set + xo[u];
-                double xv[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) xv[q] = x[c[q]];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const double s = t[u] + a[q] * xv[q];
-                    t[u] = e + q < e1 ? s : t[u];
-                }
+                for (int q = 0; q < q1; ++q) xv[u][q] = x[c[q]];
             }
+#pragma unroll
+            for (int u = 0; u < HB_RJ; ++u)
+#pragma unroll
+                for (int q = 0; q < q1; ++q) t[u] += a[q] * xv[u][q];
+        };
+        if (staged) {
+            for (; e + 4 <= e1; e += 4) add(std::integral_constant<int, 4>{}, l_val, l_col, e - t0);
+            if (e + 2 <= e1) {
+                add(std::integral_constant<int, 2>{}, l_val, l_col, e - t0);
+                e += 2;
+            }
+            if (e < e1) add(std::integral_constant<int, 1>{}, l_val, l_col, e - t0);
+        } else {
+            for (; e + 4 <= e1; e += 4) add(std::integral_constant<int, 4>{}, val, col, e);
+            for (; e < e1; ++e) add(std::integral_constant<int, 1>{}, val, col, e);
         }
         const double bi = b[i];
 #pragma unroll
         for (int u = 0; u < HB_RJ; ++u) {
             const double r = t[u] + sigma[j0 + min(u, nj - 1)] * x_set[xo[u] + i];
-            const double e1 = r - bi;
-            e2[u] += e1 * e1;
+            const double ei = r - bi;
+            e2[u] += ei * ei;
         }
         b2 += bi * bi;
     }
-#pragma unroll
-    for (int u = 0; u < HB_RJ; ++u) {
-        double e = e2[u], s2 = b2;
-        block_sum2(e, s2);
-        if (threadIdx.x == 0 && u < nj) {
-            part[((size_t)(j0 + u) * R + wg) * 2] = e;
-            part[((size_t)(j0 + u) * R + wg) * 2 + 1] = s2;
-        }
+    /* block_sum2 of every shift's pair, with one barrier */
+    __shared__ double sh[HB_RJ + 1][HB_BLOCK / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
+    static_assert(HB_RJ == 8, "two sums of four");
+    const double s0 = wave_sum4(e2[0], e2[1], e2[2], e2[3]), s1 = wave_sum4(e2[4], e2[5], e2[6], e2[7]);
+    const double sb = wave_sum2(b2, b2);
+    if ((lane & 15) == 0) {
+        const int u = (row >> 1) + 2 * (row & 1);   /* rows: the first, third, second, fourth value */
+        sh[u][wave] = s0;
+        sh[4 + u][wave] = s1;
+        if (row == 0) sh[HB_RJ][wave] = sb;
+    }
+    __syncthreads();
+    const int u = threadIdx.x;
+    if (u < nj) {
+        const double *e = sh[u], *s2 = sh[HB_RJ];
+        part[((size_t)(j0 + u) * R + wg) * 2] = ((e[0] + e[1]) + e[2]) + e[3];
+        part[((size_t)(j0 + u) * R + wg) * 2 + 1] = ((s2[0] + s2[1]) + s2[2]) + s2[3];
     }
 }
 
