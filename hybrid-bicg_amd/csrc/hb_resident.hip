@@ -68,7 +68,7 @@ template <int S, bool SOLO>
 struct res_lds {
     double rh[S][RB], s[S][RB];
     double ws[2][4 * S][4], ts[2][4 * S];
-    double x[SOLO ? S * RB : 1];   /* one workgroup: the gathered vector */
+    double x[SOLO ? S * RB + 1 : 1];   /* one workgroup: the gathered vector, and a zero */
     double ex[HB_BLOCK / 2], ep[2][HB_BLOCK / 2];
     double red[8];
     unsigned need[8];
@@ -84,6 +84,19 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
     constexpr int DP = KT & 1 ? KT / 2 : -1;
     constexpr int S = SB * E;         /* tiles of 256 rows per group of 256 threads */
     constexpr int NT = 4 * S;         /* tiles of the workgroup */
+    /* One workgroup is bound by its instructions, 16 waves on four SIMDs, so
+     * with few diagonals it keeps r^, s and the LDS address of every row's
+     * neighbour in registers: a missing entry's address is that of a zero,
+     * whose product leaves the sum as it is (the sum is never -0 and the
+     * diagonals' values are finite), and a diagonal takes a read, a product
+     * and a sum where clamping and selecting took eight more: 64 x 64, 108
+     * iterations, 967 -> 757 us. */
+    constexpr bool KEEP = SOLO && KT <= 8 && !(FULL && S * KT > 20);   /* there it spills */
+    constexpr bool PACK = S * KT > 20;   /* two 16-bit byte offsets a register */
+    /* the rows' values stay in registers where there is room: read from L2
+     * in each SpMV they were a trip of their own ahead of the sums (251 x 173,
+     * 394 iterations: 4.9 ms a solve with them kept, 5.3 without) */
+    constexpr bool VALS = FULL && KT <= 8 && (SOLO ? S * KT <= 16 : S == 1);
     auto &l_rh = L.rh;
     auto &l_s = L.s;
     auto &l_ws = L.ws;
@@ -332,7 +345,11 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
 
     /* ---- this workgroup's rows ---- */
     double r[S], p[S], q[S];
+    double k_rh[KEEP ? S : 1], k_s[KEEP ? S : 1], k_av[VALS ? S : 1][VALS ? KT : 1];
+    unsigned k_at[KEEP ? S : 1][KEEP ? PACK ? (KT + 1) / 2 : KT : 1];
     unsigned pres[S];
+    auto rh_of = [&](int sl) -> double & { return KEEP ? k_rh[KEEP ? sl : 0] : l_rh[sl][tid]; };
+    auto s_of = [&](int sl) -> double & { return KEEP ? k_s[KEEP ? sl : 0] : l_s[sl][tid]; };
     {
         const double *rs = d.rring + off((kf - 1) % (W + 1), n);
         const double *ps = fresh ? d.p_set + off(seed, n) : d.pring + off(kf % P, n);
@@ -340,16 +357,30 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
 #pragma unroll
         for (int sl = 0; sl < S; ++sl) {
             r[sl] = 0.0; p[sl] = 0.0; q[sl] = 0.0; pres[sl] = 0;
-            l_rh[sl][tid] = 0.0;
+            rh_of(sl) = 0.0;
             if (has_row(sl)) {
                 r[sl] = own(sl, rs)[ult];
                 p[sl] = own(sl, ps)[ult];
-                l_rh[sl][tid] = own(sl, (const double *)d.rhat)[ult];
+                rh_of(sl) = own(sl, (const double *)d.rhat)[ult];
                 pres[sl] = own(sl, (const unsigned short *)d.rpres)[ult];
                 if (fresh)
                     __hip_atomic_store(own(sl, pn) + ult, p[sl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            if (VALS)
+#pragma unroll
+                for (int j = 0; j < KT; ++j)
+                    k_av[VALS ? sl : 0][VALS ? j : 0] =
+                        tile_ok(sl) ? ((const double *)d.rdia + ((size_t)tile_of(sl) * KT + j) * HB_BLOCK)[ult] : 0.0;
+            if (KEEP)
+#pragma unroll
+                for (int j = 0; j < KT; ++j) {
+                    const unsigned at = 8u * (unsigned)((pres[sl] >> j) & 1u ? tile_of(sl) * HB_BLOCK + lt + d.res_off[j]
+                                                                            : S * RB);
+                    unsigned &k = k_at[KEEP ? sl : 0][KEEP ? PACK ? j / 2 : j : 0];
+                    k = PACK && j % 2 ? k | at << 16 : at;
+                }
         }
+        if (KEEP && tid == 0) l_x[S * RB] = 0.0;
     }
     /* the short last tile, T lanes per row: its group's threads take row
      * lt / T, lane lt % T */
@@ -370,6 +401,21 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
         asm volatile("" : "+v"(m));   /* its masks: anew, too */
         const double *fv = FULL ? (const double *)d.rdia + (size_t)r0 * KT : nullptr;
         double acc = 0.0;
+        if (KEEP && (T == 1 || tile_of(sl) != nblk - 1)) {
+            double xv[KT], av[FULL && !VALS ? KT : 1];
+#pragma unroll
+            for (int j = 0; j < KT; ++j) {
+                if (FULL && !VALS) av[FULL && !VALS ? j : 0] = (fv + j * HB_BLOCK)[ult];
+                unsigned k = k_at[KEEP ? sl : 0][KEEP ? PACK ? j / 2 : j : 0];
+                if (PACK) asm volatile("" : "+v"(k));   /* unpacked here, not ahead of the loop */
+                const unsigned at = !PACK ? k : j % 2 ? k >> 16 : k & 0xffffu;
+                xv[j] = *(const double *)((const char *)l_x + at);
+            }
+#pragma unroll
+            for (int j = 0; j < KT; ++j)
+                acc += (VALS ? k_av[VALS ? sl : 0][VALS ? j : 0] : FULL ? av[FULL && !VALS ? j : 0] : d.res_val[j]) * xv[j];
+            return acc;
+        }
         if (T == 1 || tile_of(sl) != nblk - 1) {
             constexpr int H = KT > 8 ? 8 : KT;
 #pragma unroll
@@ -377,7 +423,8 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
                 double xv[H], av[FULL ? H : 1];
 #pragma unroll
                 for (int j = 0; j < H; ++j)
-                    if (FULL) av[FULL ? j : 0] = (fv + (h + j) * HB_BLOCK)[ult];
+                    if (FULL)
+                        av[FULL ? j : 0] = VALS ? k_av[VALS ? sl : 0][VALS ? j : 0] : (fv + (h + j) * HB_BLOCK)[ult];
                 if (r0 + omin >= 0 && r0 + HB_BLOCK - 1 + omax < n) {
                     /* every row and diagonal of the tile lies inside x */
 #pragma unroll
@@ -486,9 +533,9 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
             pa = 0.0;
             pb = 0.0;
             const double si = t + sig * p[sl];
-            l_s[sl][tid] = si;
+            s_of(sl) = si;
             if (has_row(sl)) {
-                const double rh = l_rh[sl][tid];
+                const double rh = rh_of(sl);
                 if (snap) own(sl, (double *)d.p_snap)[ult] = p[sl];
                 pa += rh * si;
                 if (switched) {
@@ -517,7 +564,7 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
 #pragma unroll
         for (int sl = 0; sl < S; ++sl) {
             if (tile_ok(sl)) {
-                q[sl] = r[sl] + nalpha * l_s[sl][tid];
+                q[sl] = r[sl] + nalpha * s_of(sl);
                 if (SOLO) l_x[tile_of(sl) * HB_BLOCK + lt] = q[sl];
                 if (has_row(sl))
                     __hip_atomic_store(own(sl, qk) + ult, q[sl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -559,7 +606,7 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
                     if (has_row(sl)) {
                         own(sl, rk)[ult] = ri;
                         ca += ri * ri;
-                        cb += l_rh[sl][tid] * ri;
+                        cb += rh_of(sl) * ri;
                     }
                 }
             }
@@ -583,7 +630,7 @@ DEV void resident_body(const D &d, res_lds<SB * E, SOLO> &L, int w, int G)
 #pragma unroll
         for (int sl = 0; sl < S; ++sl) {
             if (tile_ok(sl)) {
-                p[sl] = shift_p(p[sl], r[sl], l_s[sl][tid], beta, pbw);
+                p[sl] = shift_p(p[sl], r[sl], s_of(sl), beta, pbw);
                 if (has_row(sl))
                     __hip_atomic_store(own(sl, pn) + ult, p[sl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
