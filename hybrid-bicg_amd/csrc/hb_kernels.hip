@@ -127,6 +127,7 @@ DEV double serial_dot(const double *x, const double *y, int n, double *lds)
  * uniform values through scalar loads.  SEED1 gathers p_set[seed], SEED2
  * gathers r_{k-1} (in rring) and s, PLAIN gathers x. */
 enum { SP_SEED1 = 0, SP_SEED2 = 1, SP_PLAIN = 2 };
+#define HB_WALK_MAX 32   /* entries of a row that one thread walks with two gathers each */
 
 /* Column panels (matrices whose columns are scattered over an x larger than
  * one XCD's L2): the SpMV runs as one launch per panel of columns, each over
@@ -469,7 +470,7 @@ DEV void spmv_body(const hb_dev &d, unsigned b, const double *__restrict__ val,
 
             constexpr int U = HB_NNZ_CAP / HB_BLOCK;
             static_assert(U * HB_BLOCK == HB_NNZ_CAP, "tile capacity");
-            if (MODE == SP_SEED2 && !UNF && T == 1 && narrow && N > 0) {
+            if (MODE == SP_SEED2 && !UNF && T == 1 && narrow == 1u && N > 0) {
                 /* One row per thread.  Values and 16-bit column offsets are
                  * staged in LDS, then each thread walks its own row: the lanes of
                  * a wave gather the same stencil slot of consecutive rows, i.e.
@@ -477,7 +478,11 @@ DEV void spmv_body(const hb_dev &d, unsigned b, const double *__restrict__ val,
                  * several cache lines per instruction.  Two gathers per entry
                  * (r and s), four entries in flight.  The row sum runs in CSR
                  * order with the products rounded on their own, as in the LDS
-                 * products path below. */
+                 * products path below.
+                 * Not where a row has more than HB_WALK_MAX entries, eight
+                 * trips of four: its thread's trips were the whole launch, 50
+                 * us on 20000 power-law rows of 31 entries on average, against
+                 * 17 with the products below */
     #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int e = tid + u * HB_BLOCK;
@@ -559,10 +564,36 @@ DEV void spmv_body(const hb_dev &d, unsigned b, const double *__restrict__ val,
                 double acc = lane == 0 ? cin : 0.0;
                 const int hi = (int)rp[row + 1];
                 int e = (int)rp[row] + lane;
-                /* a long row in a tile of many (power-law rows: two lanes for
-                 * hundreds of entries): eight reads in flight, added in order.
-                 * One read per addition took 45 us a SpMV on 60000 such rows,
-                 * most of it in the tiles that hold one */
+                /* a long row in a tile of many (power-law rows: one or two
+                 * lanes for hundreds of entries): its additions are a chain,
+                 * and the next eight reads are in flight during eight of them.
+                 * 60000 such rows, a solve: one read per addition 44.8 ms,
+                 * eight reads and then their additions 27.0, so 25.9.  Sixteen
+                 * at a time measured 24.9, but their registers cost a stencil
+                 * of 2.2M rows, which shares the kernel, a fifth. */
+                if (e + 23 * T < hi) {
+                    double v[8], w[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = prod[e + u * T];
+                    /* entries e .. are in v */
+                    for (; e + 23 * T < hi; e += 16 * T) {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) w[u] = prod[e + (8 + u) * T];
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) acc += v[u];
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) v[u] = prod[e + (16 + u) * T];
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) acc += w[u];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc += v[u];
+                    e += 8 * T;
+                }
                 for (; e + 7 * T < hi; e += 8 * T) {
                     double v[8];
 #pragma unroll
@@ -688,7 +719,8 @@ __global__ __launch_bounds__(HB_BLOCK) void k_fill(double *p, size_t count, doub
 }
 
 /* Tile b of the SpMV: col16[e] = col[e] - (tile's first row) for its
- * entries, and cflag[b] = 1 when every such offset fits in 16 bits (banded
+ * entries, and cflag[b] = 1 (3: a row has more than HB_WALK_MAX entries)
+ * when every such offset fits in 16 bits (banded
  * and stencil matrices; the SpMV then reads 2 bytes per column index).
  * Built once per plan. */
 __global__ __launch_bounds__(HB_BLOCK) void k_compress_cols(const unsigned *__restrict__ ptr,
@@ -705,8 +737,11 @@ __global__ __launch_bounds__(HB_BLOCK) void k_compress_cols(const unsigned *__re
         if (o < -32768 || o > 32767) ok = 0;
         else col16[e] = (short)o;
     }
+    const unsigned r = r0 + threadIdx.x;
+    const int lng = r < blk[b + 1] && ptr[r + 1] - ptr[r] > HB_WALK_MAX;
     ok = __syncthreads_and(ok);
-    if (threadIdx.x == 0) cflag[b] = (unsigned)ok;
+    const int any = __syncthreads_or(lng);
+    if (threadIdx.x == 0) cflag[b] = ok ? any ? 3u : 1u : 0u;
 }
 
 template <bool EXACT>

@@ -151,7 +151,8 @@ typedef struct hb_dev {
     HB_G const unsigned *ptr;
     HB_G const unsigned *blk;  /* SpMV workgroup row starts [nblk+1]       */
     HB_G const short    *col16;/* [nz] col - (first row of the entry's tile), where it fits */
-    HB_G const unsigned *cflag;      /* [nblk] 1: the tile's col16 entries are exact */
+    HB_G const unsigned *cflag;      /* [nblk] 1 or 3: the tile's col16 entries are exact;
+                                        3: and it has a row of many entries         */
     HB_G const unsigned char *vidx;  /* value table indices, tile-padded (tpad), or NULL */
     HB_G const short    *col16p;     /* col16 in the same tile-padded layout (with vidx) */
     HB_G const unsigned *tpad;       /* [nblk+1] tile b's entries start at tpad[b], a
