@@ -5,9 +5,8 @@
  * counts rows (src/matrix.c:125-187, 206-232): rows ascending, entries of one
  * row in file order.  Here the same order comes from an LSD radix sort of the
  * row indices (8-bit digits, as many passes as the row count needs), whose
- * passes are stable, carrying each entry's position; col and val are then
- * gathered through the sorted positions, and ptr[i] is the first sorted
- * position whose row is >= i (a binary search per row).
+ * passes are stable and carry col and val along, and ptr[i] is the first
+ * sorted position whose row is >= i (a binary search per row).
  *
  * One radix pass = three launches:
  *   rs_hist     per tile of RS_TILE entries, the count of each digit, stored
@@ -19,7 +18,12 @@
  *               entries and walks them 64 at a time; lanes with the same
  *               digit find each other with 8 ballots, the lowest such lane
  *               adds the group to the wavefront's LDS counter for the digit
- *               and hands the old count to its group.
+ *               and hands the old count to its group.  The tile is ordered
+ *               in LDS and written from there, a digit's entries side by side.
+ * Bound by memory: 32 bytes in and out a pass and entry.  Carrying positions
+ * instead, each entry stored where it was ranked, took 125 us a pass on 7M
+ * entries and the gather of col and val in no order 259 us at the end, 0.81
+ * ms a call; so 58 us a pass (4 TB/s) and 0.35 ms.
  * All counters are 32-bit: nz < 2^32.
  */
 #include <hip/hip_runtime.h>
@@ -69,65 +73,6 @@ __global__ __launch_bounds__(HB_BLOCK) void k_rs_hist(const unsigned *__restrict
     hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = cnt[threadIdx.x];
 }
 
-/* vals_in == NULL: the values are the entry positions 0 .. nz-1 */
-__global__ __launch_bounds__(HB_BLOCK) void k_rs_scatter(const unsigned *__restrict__ keys_in,
-                                                         const unsigned *__restrict__ vals_in,
-                                                         unsigned *__restrict__ keys_out,
-                                                         unsigned *__restrict__ vals_out,
-                                                         unsigned nz, int shift,
-                                                         const unsigned *__restrict__ offs,
-                                                         unsigned ntiles)
-{
-    __shared__ unsigned wcnt[RS_WAVES][RS_DIGITS];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-#pragma unroll
-    for (int v = 0; v < RS_WAVES; ++v) wcnt[v][tid] = 0;
-    __syncthreads();
-    const size_t wbase = (size_t)blockIdx.x * RS_TILE + (size_t)w * RS_WITEMS;
-    const u64 lt = (1ull << lane) - 1ull;
-
-    /* count each digit per wavefront */
-    for (int r = 0; r < RS_WITEMS / 64; ++r) {
-        const size_t i = wbase + (size_t)r * 64 + lane;
-        const bool valid = i < nz;
-        const unsigned d = valid ? (keys_in[i] >> shift) & (RS_DIGITS - 1) : 0u;
-        const u64 peers = same_digit(d, valid);
-        if (valid && (peers & lt) == 0) atomicAdd(&wcnt[w][d], (unsigned)__popcll(peers));
-    }
-    __syncthreads();
-    /* thread = digit: the tile's first position for the digit, then the
-     * wavefronts' shares in order */
-    {
-        unsigned run = offs[(size_t)tid * ntiles + blockIdx.x];
-#pragma unroll
-        for (int v = 0; v < RS_WAVES; ++v) {
-            const unsigned c = wcnt[v][tid];
-            wcnt[v][tid] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    /* scatter in order: the group leader takes the group's positions from the
-     * wavefront's counter and passes the first one to its group */
-    for (int r = 0; r < RS_WITEMS / 64; ++r) {
-        const size_t i = wbase + (size_t)r * 64 + lane;
-        const bool valid = i < nz;
-        const unsigned key = valid ? keys_in[i] : 0u;
-        const unsigned d = (key >> shift) & (RS_DIGITS - 1);
-        const u64 peers = same_digit(d, valid);
-        const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
-        unsigned first = 0;
-        if (valid && leader == lane) first = atomicAdd(&wcnt[w][d], (unsigned)__popcll(peers));
-        first = __shfl(first, leader, 64);
-        if (valid) {
-            const unsigned dst = first + (unsigned)__popcll(peers & lt);
-            keys_out[dst] = key;
-            vals_out[dst] = vals_in ? vals_in[i] : (unsigned)i;
-        }
-    }
-}
-
-/* ---- exclusive scan of u32 ---------------------------------------------------- */
 /* exclusive prefix of v over the workgroup; total in *tot (all threads) */
 __device__ __forceinline__ unsigned block_exscan(unsigned v, unsigned *tot)
 {
@@ -153,6 +98,104 @@ __device__ __forceinline__ unsigned block_exscan(unsigned v, unsigned *tot)
     return before + inc - v;
 }
 
+__global__ __launch_bounds__(HB_BLOCK) void k_rs_scatter(const unsigned *__restrict__ keys_in,
+                                                         const unsigned *__restrict__ cols_in,
+                                                         const double *__restrict__ vals_in,
+                                                         unsigned *__restrict__ keys_out,
+                                                         unsigned *__restrict__ cols_out,
+                                                         double *__restrict__ vals_out,
+                                                         unsigned nz, int shift,
+                                                         const unsigned *__restrict__ offs,
+                                                         unsigned ntiles)
+{
+    constexpr int PER = RS_TILE / HB_BLOCK;
+    __shared__ unsigned wcnt[RS_WAVES][RS_DIGITS], goff[RS_DIGITS];
+    __shared__ double stage[RS_TILE];   /* keys and columns, then values */
+    unsigned *l_key = (unsigned *)stage, *l_col = l_key + RS_TILE;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const size_t base = (size_t)blockIdx.x * RS_TILE;
+    const int cnt = nz - base < RS_TILE ? (int)(nz - base) : RS_TILE;
+    const int i0 = w * RS_WITEMS + lane;
+    const u64 lt = (1ull << lane) - 1ull;
+    unsigned key[PER], col[PER], pos[PER];
+    double val[PER];
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        const int i = min(i0 + 64 * r, cnt - 1);
+        key[r] = keys_in[base + i];
+    }
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        const int i = min(i0 + 64 * r, cnt - 1);
+        col[r] = cols_in[base + i];
+        val[r] = vals_in[base + i];
+    }
+#pragma unroll
+    for (int v = 0; v < RS_WAVES; ++v) wcnt[v][tid] = 0;
+    __syncthreads();
+    /* ranks among the wavefront's entries of the same digit */
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        const bool valid = i0 + 64 * r < cnt;
+        const unsigned d = (key[r] >> shift) & (RS_DIGITS - 1);
+        const u64 peers = same_digit(d, valid);
+        const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
+        unsigned first = 0;
+        if (valid && leader == lane) first = atomicAdd(&wcnt[w][d], (unsigned)__popcll(peers));
+        first = __shfl(first, leader, 64);
+        pos[r] = first + (unsigned)__popcll(peers & lt);
+    }
+    __syncthreads();
+    /* thread = digit: where the digit's entries begin in the ordered tile and
+     * in the output, then the wavefronts' shares in order */
+    {
+        unsigned c[RS_WAVES], n = 0, tot;
+#pragma unroll
+        for (int v = 0; v < RS_WAVES; ++v) {
+            c[v] = wcnt[v][tid];
+            n += c[v];
+        }
+        unsigned run = block_exscan(n, &tot);
+        goff[tid] = offs[(size_t)tid * ntiles + blockIdx.x] - run;
+#pragma unroll
+        for (int v = 0; v < RS_WAVES; ++v) {
+            wcnt[v][tid] = run;
+            run += c[v];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        if (i0 + 64 * r >= cnt) continue;
+        pos[r] += wcnt[w][(key[r] >> shift) & (RS_DIGITS - 1)];
+        l_key[pos[r]] = key[r];
+        l_col[pos[r]] = col[r];
+    }
+    __syncthreads();
+    unsigned dst[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * HB_BLOCK;
+        dst[u] = 0;
+        if (i >= cnt) continue;
+        const unsigned k = l_key[i];
+        dst[u] = goff[(k >> shift) & (RS_DIGITS - 1)] + (unsigned)i;
+        keys_out[dst[u]] = k;
+        cols_out[dst[u]] = l_col[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+        if (i0 + 64 * r < cnt) stage[pos[r]] = val[r];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * HB_BLOCK;
+        if (i < cnt) vals_out[dst[u]] = stage[i];
+    }
+}
+
+/* ---- exclusive scan of u32 ---------------------------------------------------- */
 /* bsum[b] = sum of in[b*SC_TILE .. ) */
 __global__ __launch_bounds__(HB_BLOCK) void k_scan_sums(const unsigned *__restrict__ in, size_t len,
                                                         unsigned *__restrict__ bsum)
@@ -218,17 +261,13 @@ __global__ __launch_bounds__(HB_BLOCK) void k_coo_check(const unsigned *__restri
     if (b && threadIdx.x == 0) atomicOr(bad, 1u);
 }
 
-/* ocol[e] = col[perm[e]], oval[e] = val[perm[e]] (perm NULL: identity) */
-__global__ __launch_bounds__(HB_BLOCK) void k_coo_gather(const unsigned *__restrict__ perm,
-                                                         const unsigned *__restrict__ col,
-                                                         const double *__restrict__ val, unsigned nz,
-                                                         unsigned *__restrict__ ocol,
-                                                         double *__restrict__ oval)
+__global__ __launch_bounds__(HB_BLOCK) void k_coo_copy(const unsigned *__restrict__ col,
+                                                       const double *__restrict__ val, unsigned nz,
+                                                       unsigned *__restrict__ ocol, double *__restrict__ oval)
 {
     for (size_t e = (size_t)blockIdx.x * HB_BLOCK + threadIdx.x; e < nz; e += (size_t)gridDim.x * HB_BLOCK) {
-        const unsigned s = perm ? perm[e] : (unsigned)e;
-        ocol[e] = col[s];
-        oval[e] = val[s];
+        ocol[e] = col[e];
+        oval[e] = val[e];
     }
 }
 
@@ -278,8 +317,10 @@ extern "C" int hbicg_coo2csr_device(const unsigned *row, const unsigned *col, co
     const unsigned ntiles = (unsigned)(((size_t)nz + RS_TILE - 1) / RS_TILE);
     const size_t hlen = (size_t)RS_DIGITS * ntiles;
     const size_t scan_tmp = (hlen + SC_TILE - 1) / SC_TILE + 1;
-    /* one allocation: flag, keys x2, positions x2, histogram, scan partials */
-    const size_t words = 64 + (passes ? 4 * (size_t)nz + hlen + scan_tmp : 0);
+    /* one allocation: flag, keys x2, with more than one pass columns and
+     * values (8-byte aligned), histogram, scan partials */
+    const size_t nze = (size_t)nz + (nz & 1u);
+    const size_t words = 64 + (passes ? (passes > 1 ? 5 : 2) * nze + hlen + scan_tmp : 0);
     unsigned *buf = (unsigned *)hb_pool_get(words * sizeof(unsigned));
     if (!buf) return HBICG_E_NOMEM;
     int rc = 0;
@@ -298,29 +339,37 @@ extern "C" int hbicg_coo2csr_device(const unsigned *row, const unsigned *col, co
          * order is the CSR order */
         hipLaunchKernelGGL(k_coo_ptr, dim3(grid_for((size_t)rows + 1)), dim3(HB_BLOCK), 0, s, row, nz, rows, ptr);
         if (nz > 0)
-            hipLaunchKernelGGL(k_coo_gather, dim3(grid_for(nz)), dim3(HB_BLOCK), 0, s,
-                               (const unsigned *)nullptr, col, val, nz, ocol, oval);
+            hipLaunchKernelGGL(k_coo_copy, dim3(grid_for(nz)), dim3(HB_BLOCK), 0, s, col, val, nz, ocol, oval);
     } else {
-        unsigned *k0 = buf + 64, *k1 = k0 + nz, *v0 = k1 + nz, *v1 = v0 + nz;
-        unsigned *hist = v1 + nz, *tmp = hist + hlen;
-        const unsigned *kin = row, *vin = nullptr;
-        unsigned *kout = k0, *vout = v0;
+        unsigned *k0 = buf + 64, *k1 = k0 + nze, *rest = k1 + nze;
+        unsigned *tcol = nullptr;
+        double *tval = nullptr;
+        if (passes > 1) {
+            tval = (double *)rest;
+            tcol = rest + 2 * nze;
+            rest = tcol + nze;
+        }
+        unsigned *hist = rest, *tmp = hist + hlen;
+        const unsigned *kin = row, *cin = col;
+        const double *vin = val;
+        unsigned *kout = k0;
         for (int p = 0; p < passes && e == hipSuccess; ++p) {
             const int shift = p * RS_BITS;
+            /* the last pass, and every other one before it, into the output */
+            unsigned *cout = (passes - 1 - p) & 1 ? tcol : ocol;
+            double *vout = (passes - 1 - p) & 1 ? tval : oval;
             hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(HB_BLOCK), 0, s, kin, nz, shift, hist, ntiles);
             e = scan_u32(hist, hist, hlen, tmp, s);
             if (e != hipSuccess) break;
-            hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(HB_BLOCK), 0, s, kin, vin, kout, vout, nz,
+            hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(HB_BLOCK), 0, s, kin, cin, vin, kout, cout, vout, nz,
                                shift, (const unsigned *)hist, ntiles);
             kin = kout;
+            cin = cout;
             vin = vout;
             kout = (kout == k0) ? k1 : k0;
-            vout = (vout == v0) ? v1 : v0;
         }
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_coo_gather, dim3(grid_for(nz)), dim3(HB_BLOCK), 0, s, vin, col, val, nz, ocol, oval);
+        if (e == hipSuccess)
             hipLaunchKernelGGL(k_coo_ptr, dim3(grid_for((size_t)rows + 1)), dim3(HB_BLOCK), 0, s, kin, nz, rows, ptr);
-        }
     }
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s);

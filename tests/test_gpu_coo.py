@@ -179,3 +179,13 @@ def test_matrix_market_file_to_device_solve(tmp_path):
             L.hbicg_plan_destroy(pl)
     finally:
         L.hbicg_csr_free_device(C.byref(csr))
+
+
+@pytest.mark.parametrize("rows", [2, 256, 257, 65_537])      # one, one, two and three passes
+@pytest.mark.parametrize("nz", [1, 63, 64, 65, 4095, 4096, 4097, 8191])
+def test_tile_edges(rows, nz):
+    """Entries around a wavefront's 64 and a tile's 4096, odd counts, every number of passes."""
+    rng = np.random.default_rng(nz)
+    row = rng.integers(0, rows, nz).astype(np.uint32)
+    row[0] = rows - 1
+    _check(rows, row, rng.integers(0, min(rows, 50), nz).astype(np.uint32), rng.standard_normal(nz))
