@@ -974,6 +974,7 @@ static hbicg_plan *plan_create_v(const hbicg_csr *A, int a_on_device, int M,
 
     /* alpha~'s finalize joins SpMV 2 where that launch forms q at its
      * gathered columns in one pass */
+    d->fused_q = d->fused && d->q_unfused && (p->fused == 1 || p->fused == 3 || p->fused == 4);
     d->fused_a = d->fused && !d->q_unfused && d->npanel <= 1 && (p->fused == 1 || p->fused == 3 || p->fused == 4);
     /* the scalar stage joins the shift kernel (level 1), whose tiles then
      * walk the seed p update and the flush tiles grid-stride */

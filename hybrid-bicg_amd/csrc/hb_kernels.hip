@@ -818,6 +818,29 @@ __global__ __launch_bounds__(HB_BLOCK) void k_fin_spmv(hb_dev d)
     fin_spmv_body<MODE, EXACT>(d);
 }
 
+/* k_qform with alpha~'s finalize as the launch's first workgroup: one launch
+ * fewer an iteration where q is formed before SpMV 2 (60000 power-law rows,
+ * 414 iterations: 26.0 -> 25.2 ms). */
+__global__ __launch_bounds__(HB_BLOCK) void k_qform_fa(hb_dev d)
+{
+    if (blockIdx.x == 0) {
+        fin_spmv_body<SP_SEED1, false, true>(d);
+        return;
+    }
+    hb_state *st = d.st;
+    const int done = st->done, k = st->k;
+    if (done | (k < 1)) return;
+    const int n = d.n, stride = (gridDim.x - 1) * HB_BLOCK;
+    const double *__restrict__ r = d.rring + off((k - 1) % (d.W + 1), n);
+    const double *__restrict__ s = d.s;
+    double *__restrict__ q = d.qring + off(k % d.W, n);
+    int i = (blockIdx.x - 1) * HB_BLOCK + threadIdx.x;
+    const double r0 = r[min(i, n - 1)], s0 = s[min(i, n - 1)];   /* on their way during the wait */
+    const double nalpha = -mail_wait(&st->mail_a, st);
+    if (i < n) q[i] = r0 + nalpha * s0;
+    for (i += stride; i < n; i += stride) q[i] = r[i] + nalpha * s[i];
+}
+
 /* Fused SpMV 2 (default mode, q formed at the gathered columns): workgroup
  * 0 finalizes alpha~ from SpMV 1's partials and publishes it; the others
  * are the tiles, which issue their loads and gathers first and read alpha~
@@ -3033,15 +3056,22 @@ static int stage_fused(const hb_dev *d, int stage, hipStream_t s)
     return (int)hipGetLastError();
 }
 
+static void launch_qform(const hb_dev *d, hipStream_t s)
+{
+    if (d->fused_q) hipLaunchKernelGGL(k_qform_fa, dim3(d->vec_grid + 1), dim3(HB_BLOCK), 0, s, *d);
+    else hipLaunchKernelGGL(k_qform, dim3(d->vec_grid), dim3(HB_BLOCK), 0, s, *d);
+}
+
 int hb_k_stage(const hb_dev *d, int stage, hipStream_t s)
 {
     const dim3 gs(d->nblk), gv(d->vec_grid), bl(HB_BLOCK), one(1);
+    if (d->fused_q && stage == HB_STAGE_FIN1) return 0;
     if (d->fused && !d->exact &&
         (stage == HB_STAGE_FIN2 || stage == HB_STAGE_SEED || stage == HB_STAGE_COEF || stage == HB_STAGE_SHIFT ||
          stage == HB_STAGE_SCALAR || (d->fused_a && (stage == HB_STAGE_FIN1 || stage == HB_STAGE_SPMV2))))
         return stage_fused(d, stage, s);
     if (d->npanel > 1 && (stage == HB_STAGE_SPMV1 || stage == HB_STAGE_SPMV2)) {
-        if (stage == HB_STAGE_SPMV2 && d->q_unfused) hipLaunchKernelGGL(k_qform, gv, bl, 0, s, *d);
+        if (stage == HB_STAGE_SPMV2 && d->q_unfused) launch_qform(d, s);
         if (stage == HB_STAGE_SPMV1) {
             if (d->exact) spmv_panels<SP_SEED1, true, false>(d, s);
             else spmv_panels<SP_SEED1, false, false>(d, s);
@@ -3072,7 +3102,7 @@ int hb_k_stage(const hb_dev *d, int stage, hipStream_t s)
         break;
     case HB_STAGE_SPMV2:
         if (d->q_unfused && !d->exact) {
-            hipLaunchKernelGGL(k_qform, gv, bl, 0, s, *d);
+            launch_qform(d, s);
             if (d->cdia) hipLaunchKernelGGL((k_spmv<SP_SEED2, false, true, true, true>), gs, bl, 0, s, *d);
             else if (d->vidx) hipLaunchKernelGGL((k_spmv<SP_SEED2, false, true, true>), gs, bl, 0, s, *d);
             else hipLaunchKernelGGL((k_spmv<SP_SEED2, false, false, true>), gs, bl, 0, s, *d);
@@ -3134,7 +3164,7 @@ int hb_k_stage_runs(const hb_dev *d, int stage)
     if (stage == HB_STAGE_COEF) return !d->exact && !d->fused;
     if (d->exact || !d->fused) return 1;
     if (stage == HB_STAGE_FIN2) return 0;
-    if (stage == HB_STAGE_FIN1) return !d->fused_a;
+    if (stage == HB_STAGE_FIN1) return !d->fused_a && !d->fused_q;
     if (stage == HB_STAGE_SCALAR) return !d->fused_s;
     return 1;
 }

@@ -179,6 +179,8 @@ typedef struct hb_dev {
     unsigned pboff[HB_MAXPANEL];
     int npart;                       /* partial-sum pairs the seed SpMVs write: nblk, or
                                         the last panel's tile count                    */
+    int fused_q;                     /* the alpha~ finalize runs as the first workgroup of
+                                        the launch that forms q ahead of SpMV 2        */
     int fused_a;                     /* the alpha~ finalize runs as SpMV 2's first
                                         workgroup (fused launches, q formed at the
                                         gathered columns, one pass)                    */

@@ -92,7 +92,8 @@ typedef struct hbicg_params {
                             Elsewhere four launches per iteration --
                             the alpha~ finalize runs as the first workgroup of SpMV
                             2's launch (where SpMV 2 forms q at its gathered columns
-                            in one pass; else it keeps its own launch), the omega~
+                            in one pass; of the launch that forms q where one does;
+                            else it keeps its own launch), the omega~
                             finalize as the first workgroup of the seed update's, the
                             scalar stage as the first workgroup of the shift kernel's
                             (beta~ handed to the seed p update as soon as it is
@@ -104,8 +105,9 @@ typedef struct hbicg_params {
                             as in 3); 3: the same with the scalar stage in a launch
                             of its own (five launches); 2: also alpha~ on its own
                             (six); 0: eight launches.  Same results bit for bit; the
-                            batched solver always uses eight, exact order seven (no
-                            coefficient kernel)                                         */
+                            batched solver uses the resident form where all its
+                            problems fit it and eight launches elsewhere, exact order
+                            seven (no coefficient kernel)                              */
     int    panel_cols;   /* seed SpMVs in column panels of this many columns: one pass
                             per panel over the entries whose columns lie in it, row sums
                             carried between passes, so the gathers of a pass stay within
